@@ -55,12 +55,15 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) {
   return __uint_as_float(static_cast<uint32_t>(b) << 16);
 }
 
-// fp32 -> bf16 with round-to-nearest-even; NaN stays a quiet NaN.
+// fp32 -> bf16 with round-to-nearest-even; NaN stays a quiet NaN.  The
+// conversion instruction (v_cvt_pk_bf16_f32): bit for bit the integer form
+// (add 0x7fff plus the low kept bit, shift, NaN aside), compared on the card
+// over all 2^32 inputs.  One instruction for about seven: the decode kernels
+// run most of their code once a wave, so they wait for its fetch (one decoder
+// layer in a hipGraph, 5 tokens: 62.8 -> 52.8 us; 64 tokens with the lm_head:
+// 125.9 -> 114.2; 24 layers of short-context attention: 144.5 -> 138.9).
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
 __device__ __forceinline__ float load_as_f32(const void *p, int64_t i, int dtype) {

@@ -59,6 +59,23 @@ def test_add_rmsnorm_matches_qwen2_rmsnorm(gpu, with_delta, hidden, dtype):
         torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-6)
 
 
+def test_bf16_rounding_of_any_value(gpu):
+    """fp32 -> bf16 in the kernels on sums of arbitrary bf16 bit patterns:
+    subnormals, ties, overflow to infinity, infinities and NaN (exact but for
+    a NaN's payload)."""
+    g = torch.Generator(device=gpu).manual_seed(2)
+    draw = lambda: torch.randint(-2**15, 2**15, (512, 896), generator=g, device=gpu, dtype=torch.int16)
+    h, d = draw(), draw()
+    d[::2] = (h[::2] & ~0x7f) - (draw()[::2] & 0xfff)  # near h: cancellation, ties
+    h, d = h.view(torch.bfloat16), d.view(torch.bfloat16)
+    want, hk = h + d, h.clone()
+    add_rmsnorm(hk, d, torch.ones(896, device=gpu, dtype=torch.bfloat16), 1e-6)
+    nan = want.isnan()
+    assert nan.any() and want.isinf().any()
+    assert torch.equal(hk.isnan(), nan)
+    assert torch.equal(hk.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_embed_rmsnorm_matches_embedding_then_norm(gpu, dtype):
     """h = embedding rows broadcast over T (exact); x = Qwen2RMSNorm(h) to one
