@@ -165,6 +165,40 @@ int spk_decode_attn_combine(const float *partials, size_t partials_bytes, int nu
                             int head_dim, void *stream);
 
 /*
+ * Causal attention of prefill chunks on packed spikes: query i of a chunk
+ * (position ctx + i of its sequence) attends to positions 0..ctx + i.  Replaces
+ * the unpack-gather + SDPA with an offset causal mask of
+ * spikeinfer/attention.py:161-178, all chunks of a step in one launch (32 a
+ * launch).
+ *
+ *   q        int32 words of (t, batch row, query head) at q_strides, W words
+ *            contiguous; W = ceil(head_dim / 32)
+ *   k, v     int32 words of (t, kv head, slot) at kv_strides, the same for both
+ *   chunks   host array: rows [start, start + q_len) of q and out; `table` is the
+ *            sequence's block-table row on the device (n_table entries at
+ *            table_stride), key j in slot table[j/bs]*bs + j%bs, positions past
+ *            the table or whose block lies outside the cache read as zero spikes;
+ *            `table` NULL (ctx must be 0): key j is slot start + j of k and v
+ *   out      out_dtype (F32/F16/BF16) [t, batch row, query head, channel] at
+ *            out_strides, channel stride 1
+ * head_dim <= 128 (SPK_EUNSUPPORTED beyond), scale * head_dim <= 12.
+ */
+typedef struct SpkPrefillChunk {
+  int64_t start;
+  const int32_t *table;
+  int64_t table_stride;
+  int n_table;
+  int q_len;
+  int ctx;
+  int pad;
+} SpkPrefillChunk;
+int spk_prefill_attn(const int32_t *q, const int64_t q_strides[3], const int32_t *k,
+                     const int32_t *v, const int64_t kv_strides[3], int64_t num_slots,
+                     const SpkPrefillChunk *chunks, int nchunks, void *out, int out_dtype,
+                     const int64_t out_strides[3], int T, int Hq, int Hkv, int head_dim,
+                     int block_size, float scale, void *stream);
+
+/*
  * Prefill reader: one sequence's first seq_len cached tokens as dense 0/1
  * spikes, K and V in one launch.  Replaces gather_kv_unpacked
  * (spikeinfer/kernels/spike_attention.py:224-244: slot-matrix index_select,
@@ -397,6 +431,21 @@ int spk_qkv_rope_lif_pack(const void *x, int x_dtype, const int64_t x_strides[2]
                           const int64_t *slot_mapping, int64_t num_slots, void *dense_q,
                           void *dense_k, void *dense_v, int T, int64_t n_tok, int Hq,
                           int Hkv, int D, void *stream);
+
+/*
+ * The same with the step's own k and v words also written to k_packed and
+ * v_packed, int32 [T, n_tok, Hkv, W] contiguous (both or neither): the keys of a
+ * fresh chunk for spk_prefill_attn, whatever slots its tokens have.
+ */
+int spk_qkv_rope_lif_pack_kv(const void *x, int x_dtype, const int64_t x_strides[2],
+                             const void *cos, const void *sin, const int64_t *positions,
+                             int64_t table_rows, const void *beta,
+                             const void *threshold, int param_dtype, int32_t *q_packed,
+                             const int64_t q_strides[3], int64_t n_q, int32_t *k_cache,
+                             int32_t *v_cache, const int64_t cache_strides[3],
+                             const int64_t *slot_mapping, int64_t num_slots, int32_t *k_packed,
+                             int32_t *v_packed, void *dense_q, void *dense_k, void *dense_v,
+                             int T, int64_t n_tok, int Hq, int Hkv, int D, void *stream);
 
 /*
  * MLP gate: x [T, rows, 2*I] (gate in columns [0, I), up in [I, 2I); strides

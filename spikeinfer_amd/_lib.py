@@ -57,6 +57,14 @@ def pack_lif_site(x, x_strides, beta, threshold, param_dtype, scatter, out, out_
                              *out_strides, num_slots, n_tok, H, D)
 
 
+_CHUNK_FORMAT = struct.Struct("<qQqiiii")  # SpkPrefillChunk, field by field (no padding)
+
+
+def pack_prefill_chunk(start, table, table_stride, n_table, q_len, ctx) -> bytes:
+    """The bytes of one SpkPrefillChunk (``table`` 0: contiguous keys)."""
+    return _CHUNK_FORMAT.pack(start, table, table_stride, n_table, q_len, ctx, 0)
+
+
 # name -> (restype, argtypes); mirrors include/spikeinfer_amd.h
 _SIGNATURES = {
     "spk_last_error": (ctypes.c_char_p, []),
@@ -73,6 +81,9 @@ _SIGNATURES = {
         _i32, _i32, _i32, _f32, _i32, _vp, _sz, _vp]),
     "spk_decode_attn_combine": (_i32, [
         _vp, _sz, _i32, _i32, _vp, _vp, _i32, _i64p, _i32, _i32, _i32, _i32, _vp]),
+    "spk_prefill_attn": (_i32, [
+        _vp, _i64p, _vp, _vp, _i64p, _i64, ctypes.c_char_p, _i32, _vp, _i32, _i64p, _i32, _i32, _i32,
+        _i32, _i32, _f32, _vp]),
     "spk_gather_unpack": (_i32, [
         _vp, _vp, _i64p, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "spk_qkv_decode_attn": (_i32, [
@@ -96,6 +107,9 @@ _SIGNATURES = {
     "spk_qkv_rope_lif_pack": (_i32, [
         _vp, _i32, _i64p, _vp, _vp, _vp, _i64, _vp, _vp, _i32, _vp, _i64p, _i64, _vp, _vp, _i64p, _vp,
         _i64, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp]),
+    "spk_qkv_rope_lif_pack_kv": (_i32, [
+        _vp, _i32, _i64p, _vp, _vp, _vp, _i64, _vp, _vp, _i32, _vp, _i64p, _i64, _vp, _vp, _i64p, _vp,
+        _i64, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp]),
     "spk_lif_gate_mul": (_i32, [_vp, _i32, _i64p, _vp, _vp, _i32, _vp, _i32, _i64, _i32, _vp]),
     "spk_mlp_gate_packed_bytes": (_sz, [_i32, _i32]),
     "spk_linear_pack": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp]),

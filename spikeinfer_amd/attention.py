@@ -3,8 +3,8 @@
 ``paged_attention`` keeps the reference's contract (spikeinfer/attention.py:111-180):
 dense 0/1 spikes in, the step's K/V packed and scattered into the cache at
 ``meta.slot_mapping`` first, decode tokens (a contiguous prefix of the batch) through
-the popcount decode kernel, prefill chunks through unpack-gather + SDPA with a causal
-mask offset by the cached prefix, output ``[T, 1, n_tok, H_q * D]`` in the spikes'
+the popcount decode kernel, prefill chunks through the packed causal kernel (head_dim up
+to 128; unpack-gather + SDPA with an offset causal mask beyond), output ``[T, 1, n_tok, H_q * D]`` in the spikes'
 dtype.
 
 ``paged_attention_fused`` is the same step starting one stage earlier, from the LIF
@@ -21,7 +21,8 @@ import torch.nn.functional as F
 
 from .kernels.lif import lif_multistep, lif_pack_write_sites
 from .kernels.packing import pack_spikes, packed_width
-from .kernels.spike_attention import gather_kv_unpacked_pair, paged_spike_attn_decode
+from .kernels.spike_attention import (gather_kv_unpacked_pair, paged_spike_attn_decode,
+                                      paged_spike_attn_prefill, prefill_supported)
 
 
 @dataclass
@@ -81,10 +82,20 @@ def _causal_offset_mask(query_len: int, total_len: int, device, dtype) -> torch.
     return torch.triu(mask, diagonal=ctx + 1)
 
 
-def _prefill(q_dense, k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim):
+def _prefill_packed(q_packed, first, k_cache, v_cache, meta, out, head_dim):
     """Each prefill chunk attends to its sequence's whole cached prefix plus
-    itself: one gather-unpack launch yields dense K and V, then SDPA with the
-    offset causal mask (spikeinfer/attention.py:161-178)."""
+    itself, straight from the packed words (spikeinfer/attention.py:161-178).
+    Row ``i`` of ``q_packed [T, n, H_q, W]`` is batch row ``first + i``."""
+    chunks = [(start - first, start, q_len, ctx, table) for start, q_len, ctx, table in
+              zip(meta.prefill_query_starts, meta.prefill_query_lens, meta.prefill_context_lens,
+                  meta.prefill_block_tables)]
+    paged_spike_attn_prefill(q_packed, k_cache, v_cache, chunks, out, head_dim, meta.block_size)
+
+
+def _prefill(q_dense, k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim):
+    """The same from dense query spikes: one gather-unpack launch yields dense K
+    and V, then SDPA with the offset causal mask.  For what the packed kernel
+    does not take (head_dim over 128) and for gradients to dense queries."""
     dtype, device = q_dense.dtype, q_dense.device
     for i in range(meta.num_prefills):
         start = meta.prefill_query_starts[i]
@@ -124,14 +135,20 @@ def paged_attention(
     v_cache.index_copy_(2, meta.slot_mapping, pack_spikes(v_spk.squeeze(1)))
     out = torch.empty((T, n_tok, num_q_heads, head_dim), device=device, dtype=dtype)
     n_dec = meta.num_decode_tokens
+    packed = bool(meta.num_prefills) and prefill_supported(head_dim, dtype) and \
+        not (q_spk.requires_grad and torch.is_grad_enabled())
+    if packed:  # every token's query words at once: [T, n_tok, H_q, W]
+        q_words = pack_spikes(q_spk[:, 0]).permute(0, 2, 1, 3)
     if n_dec:
         q_dec = q_spk[:, 0, :, :n_dec, :].permute(0, 2, 1, 3)  # [T, n_dec, H_q, D]
         paged_spike_attn_decode(
-            pack_spikes(q_dec), k_cache, v_cache, meta.block_tables, meta.seq_lens,
-            head_dim=head_dim, block_size=meta.block_size, num_q_heads=num_q_heads,
+            q_words[:, :n_dec] if packed else pack_spikes(q_dec), k_cache, v_cache, meta.block_tables,
+            meta.seq_lens, head_dim=head_dim, block_size=meta.block_size, num_q_heads=num_q_heads,
             num_kv_heads=num_kv_heads, out=out[:, :n_dec],
         )
-    if meta.num_prefills:
+    if packed:
+        _prefill_packed(q_words, 0, k_cache, v_cache, meta, out, head_dim)
+    elif meta.num_prefills:
         _prefill(q_spk[:, 0], k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim)
     return out.view(T, 1, n_tok, num_q_heads * head_dim)
 
@@ -174,14 +191,19 @@ def paged_attention_fused(
     if out is None:
         out = torch.empty((T, n_tok, num_q_heads, head_dim), device=device, dtype=dtype)
     n_dec = meta.num_decode_tokens
-    # One launch for the three LIF sites: k and v into their cache slots, the
-    # decode tokens' q into the packed-query buffer.
+    # One launch for the LIF sites: k and v into their cache slots, the decode
+    # tokens' q into the packed-query buffer, the prefill tokens' q into another.
     sites = [(k_cur, lif_k[0], lif_k[1], k_cache, True), (v_cur, lif_v[0], lif_v[1], v_cache, True)]
     if n_dec:
         if q_packed is None:
             q_packed = torch.empty((T, n_dec, num_q_heads, packed_width(head_dim)),
                                    dtype=torch.int32, device=device)
         sites.append((q_cur[:, :n_dec], lif_q[0], lif_q[1], q_packed, False))
+    packed = bool(meta.num_prefills) and prefill_supported(head_dim, dtype)
+    if packed:
+        q_words = torch.empty((T, n_tok - n_dec, num_q_heads, packed_width(head_dim)), dtype=torch.int32,
+                              device=device)
+        sites.append((q_cur[:, n_dec:], lif_q[0], lif_q[1], q_words, False))
     lif_pack_write_sites(sites, meta.slot_mapping)
     if n_dec:
         paged_spike_attn_decode(
@@ -189,7 +211,9 @@ def paged_attention_fused(
             head_dim=head_dim, block_size=meta.block_size, num_q_heads=num_q_heads,
             num_kv_heads=num_kv_heads, out=out[:, :n_dec],
         )
-    if meta.num_prefills:
+    if packed:
+        _prefill_packed(q_words, n_dec, k_cache, v_cache, meta, out, head_dim)
+    elif meta.num_prefills:
         # Prefill queries need dense spikes for SDPA; the LIF is per token, so
         # running it on the prefill tokens alone gives the same spikes.
         q_pre = lif_multistep(q_cur[:, n_dec:], lif_q[0], lif_q[1])  # [T, n_pre, H_q, D]

@@ -407,6 +407,7 @@ struct QkvParams {
   int64_t cs0, cs1, cs2;
   const int64_t *slots;
   int64_t num_slots;
+  uint64_t *own[2];        // optional [T, n_tok, Hkv, W] contiguous k and v words of the step
   void *dense[3];          // optional [T, H, n_tok, D] spikes per site
   int T;
   int64_t n_tok;
@@ -455,7 +456,7 @@ __global__ __launch_bounds__(256) void qkv_rope_lif_pack_vec_kernel(QkvParams p)
   }
 
   // Destination of this row's packed words.
-  uint64_t *dst = nullptr;
+  uint64_t *dst = nullptr, *own = nullptr;
   int64_t dstep = 0;  // per timestep, in uint64 words
   if (active) {
     if (site == 0) {
@@ -469,8 +470,10 @@ __global__ __launch_bounds__(256) void qkv_rope_lif_pack_vec_kernel(QkvParams p)
         dst = (site == 1 ? p.k_cache : p.v_cache) + (h * p.cs1 + slot * p.cs2) / 2;
         dstep = p.cs0 / 2;
       }
+      if (p.own[site - 1]) own = p.own[site - 1] + (tok * p.Hkv + h) * (p.D >> 6);
     }
   }
+  const int64_t ostep = p.n_tok * p.Hkv * (p.D >> 6);
   E *dense = active ? static_cast<E *>(p.dense[site]) : nullptr;
   const int Hs = site == 0 ? p.Hq : p.Hkv;
   const int64_t dense_row = (static_cast<int64_t>(h) * p.n_tok + tok) * p.D + cl;
@@ -522,6 +525,7 @@ __global__ __launch_bounds__(256) void qkv_rope_lif_pack_vec_kernel(QkvParams p)
         hi |= __shfl_xor(hi, off);
       }
       if (dst && s8 == 0) dst[t * dstep + (sub >> 3)] = (static_cast<uint64_t>(hi) << 32) | lo;
+      if (own && s8 == 0) own[t * ostep + (sub >> 3)] = (static_cast<uint64_t>(hi) << 32) | lo;
       if (dense) *reinterpret_cast<Vec *>(dense + t * dense_tstep + dense_row) = spk;
     }
   }
@@ -582,7 +586,7 @@ __global__ __launch_bounds__(256) void qkv_rope_lif_pack_kernel(QkvParams p) {
   }
 
   // Destination of this row's packed words (D/64 per timestep).
-  uint64_t *dst = nullptr;
+  uint64_t *dst = nullptr, *own = nullptr;
   int64_t dstep = 0;  // per timestep, in uint64 words
   if (active) {
     if (site == 0) {
@@ -596,8 +600,10 @@ __global__ __launch_bounds__(256) void qkv_rope_lif_pack_kernel(QkvParams p) {
         dst = (site == 1 ? p.k_cache : p.v_cache) + (h * p.cs1 + slot * p.cs2) / 2;
         dstep = p.cs0 / 2;
       }
+      if (p.own[site - 1]) own = p.own[site - 1] + (tok * p.Hkv + h) * (p.D >> 6);
     }
   }
+  const int64_t ostep = p.n_tok * p.Hkv * (p.D >> 6);
   E *dense = active ? static_cast<E *>(p.dense[site]) : nullptr;
   const int Hs = site == 0 ? p.Hq : p.Hkv;
   const int64_t dense_row = (static_cast<int64_t>(h) * p.n_tok + tok) * p.D;
@@ -632,14 +638,16 @@ __global__ __launch_bounds__(256) void qkv_rope_lif_pack_kernel(QkvParams p) {
         const bool sl = lif_step(ulo[j], lo, blo[j], tlo[j]);
         const bool sh = lif_step(uhi[j], hi, bhi[j], thi[j]);
         const uint64_t ml = __ballot(sl), mh = __ballot(sh);
-        if (dst && sub == 0) {
+        auto put = [&](uint64_t *d) {
           if (R == 32) {
-            dst[t * dstep] = ((ml >> rshift) & 0xffffffffull) | (((mh >> rshift) & 0xffffffffull) << 32);
+            d[0] = ((ml >> rshift) & 0xffffffffull) | (((mh >> rshift) & 0xffffffffull) << 32);
           } else {
-            dst[t * dstep + j] = ml;
-            dst[t * dstep + P + j] = mh;
+            d[j] = ml;
+            d[P + j] = mh;
           }
-        }
+        };
+        if (dst && sub == 0) put(dst + t * dstep);
+        if (own && sub == 0) put(own + t * ostep);
         if (dense) {
           dense[t * dense_tstep + dense_row + sub + R * j] = spike_elem<DT>(sl);
           dense[t * dense_tstep + dense_row + sub + R * j + half] = spike_elem<DT>(sh);
@@ -871,14 +879,14 @@ extern "C" int spk_rmsnorm_mean_t(const void *h, const void *delta, const void *
   return check_launch("rmsnorm_mean_t");
 }
 
-extern "C" int spk_qkv_rope_lif_pack(
+extern "C" int spk_qkv_rope_lif_pack_kv(
     const void *x, int x_dtype, const int64_t x_strides[2], const void *cos, const void *sin,
     const int64_t *positions, int64_t table_rows,
     const void *beta, const void *threshold, int param_dtype, int32_t *q_packed,
     const int64_t q_strides[3], int64_t n_q, int32_t *k_cache, int32_t *v_cache,
     const int64_t cache_strides[3], const int64_t *slot_mapping, int64_t num_slots,
-    void *dense_q, void *dense_k, void *dense_v, int T, int64_t n_tok, int Hq, int Hkv, int D,
-    void *stream) {
+    int32_t *k_packed, int32_t *v_packed, void *dense_q, void *dense_k, void *dense_v, int T,
+    int64_t n_tok, int Hq, int Hkv, int D, void *stream) {
   if (x_dtype != SPK_BF16 && x_dtype != SPK_F16)
     return fail(SPK_EUNSUPPORTED, "qkv_rope_lif_pack: input dtype %d (bf16 or f16 only)", x_dtype);
   if (!valid_float_dtype(param_dtype))
@@ -900,6 +908,9 @@ extern "C" int spk_qkv_rope_lif_pack(
   if (n_q > 0 && ((reinterpret_cast<uintptr_t>(q_packed) & 7) ||
                   ((q_strides[0] | q_strides[1] | q_strides[2]) & 1)))
     return fail(SPK_EINVAL, "qkv_rope_lif_pack: q buffer must be 8-byte aligned with even strides");
+  if ((k_packed == nullptr) != (v_packed == nullptr) ||
+      ((reinterpret_cast<uintptr_t>(k_packed) | reinterpret_cast<uintptr_t>(v_packed)) & 7))
+    return fail(SPK_EINVAL, "qkv_rope_lif_pack: k_packed and v_packed go together, 8-byte aligned");
   void *dense[3] = {dense_q, dense_k, dense_v};
   for (void *d : dense)
     if (d && !aligned16(d)) return fail(SPK_EINVAL, "qkv_rope_lif_pack: dense outputs must be 16-byte aligned");
@@ -929,6 +940,8 @@ extern "C" int spk_qkv_rope_lif_pack(
   p.cs2 = cache_strides[2];
   p.slots = slot_mapping;
   p.num_slots = num_slots;
+  p.own[0] = reinterpret_cast<uint64_t *>(k_packed);
+  p.own[1] = reinterpret_cast<uint64_t *>(v_packed);
   for (int i = 0; i < 3; ++i) p.dense[i] = dense[i];
   p.T = T;
   p.n_tok = n_tok;
@@ -952,6 +965,20 @@ extern "C" int spk_qkv_rope_lif_pack(
       qkv_rope_lif_pack_kernel<SPK_F16><<<grid, 256, 0, s>>>(p);
   }
   return check_launch("qkv_rope_lif_pack");
+}
+
+extern "C" int spk_qkv_rope_lif_pack(
+    const void *x, int x_dtype, const int64_t x_strides[2], const void *cos, const void *sin,
+    const int64_t *positions, int64_t table_rows,
+    const void *beta, const void *threshold, int param_dtype, int32_t *q_packed,
+    const int64_t q_strides[3], int64_t n_q, int32_t *k_cache, int32_t *v_cache,
+    const int64_t cache_strides[3], const int64_t *slot_mapping, int64_t num_slots,
+    void *dense_q, void *dense_k, void *dense_v, int T, int64_t n_tok, int Hq, int Hkv, int D,
+    void *stream) {
+  return spk_qkv_rope_lif_pack_kv(x, x_dtype, x_strides, cos, sin, positions, table_rows, beta, threshold,
+                                  param_dtype, q_packed, q_strides, n_q, k_cache, v_cache, cache_strides,
+                                  slot_mapping, num_slots, nullptr, nullptr, dense_q, dense_k, dense_v, T,
+                                  n_tok, Hq, Hkv, D, stream);
 }
 
 extern "C" int spk_lif_gate_mul(const void *x, int dtype, const int64_t x_strides[2],

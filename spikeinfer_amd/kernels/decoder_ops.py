@@ -126,6 +126,7 @@ def qkv_rope_lif_pack(
     n_q: int = 0,
     dense: tuple[torch.Tensor | None, torch.Tensor | None, torch.Tensor | None] | None = None,
     positions: torch.Tensor | None = None,
+    kv_packed: tuple[torch.Tensor, torch.Tensor] | None = None,
 ) -> torch.Tensor | None:
     """RoPE -> LIF -> pack for the q/k/v site of one layer.
 
@@ -140,6 +141,8 @@ def qkv_rope_lif_pack(
             token ``i`` is written at ``slot_mapping[i]``.
         q_packed: ``int32 [T, n_q, Hq, W]`` receiving tokens ``[0, n_q)``.
         dense: optional ``[T, H, n_tok, D]`` outputs of the 0/1 spikes per site.
+        kv_packed: optional contiguous ``int32 [T, n_tok, Hkv, W]`` pair that
+            receives the k and v words too, token by token.
     Returns ``q_packed``.
     """
     dev = _lib.require_gpu(qkv, cos, sin, beta, threshold, k_cache, v_cache, slot_mapping, q_packed,
@@ -178,16 +181,22 @@ def qkv_rope_lif_pack(
         if t is not None and (tuple(t.shape) != (T, H, n_tok, head_dim) or not t.is_contiguous()
                               or t.dtype != qkv.dtype):
             raise ValueError(f"dense spikes must be contiguous [T, {H}, {n_tok}, {head_dim}] {qkv.dtype}")
+    pk, pv = kv_packed if kv_packed is not None else (None, None)
+    for t in (pk, pv):
+        if t is not None and (tuple(t.shape) != (T, n_tok, num_kv_heads, head_dim // 32) or
+                              t.dtype != torch.int32 or not t.is_contiguous() or t.device != dev):
+            raise ValueError(f"kv_packed must be contiguous int32 [{T}, {n_tok}, {num_kv_heads}, W]")
     if k_cache.shape != v_cache.shape or k_cache.stride() != v_cache.stride():
         raise ValueError("k and v caches must have the same shape and strides")
     _lib.check(
-        _lib.load().spk_qkv_rope_lif_pack(
+        _lib.load().spk_qkv_rope_lif_pack_kv(
             qkv.data_ptr(), _lib.dtype_code(qkv.dtype), (_lib.ctypes.c_int64 * 2)(*qkv.stride()[:2]),
             cos.data_ptr(), sin.data_ptr(), _lib.ptr(positions), rows if positions is not None else 0,
             beta.data_ptr(), threshold.data_ptr(),
             _lib.dtype_code(beta.dtype), _lib.ptr(q_packed), qs, n_q,
             k_cache.data_ptr(), v_cache.data_ptr(), (_lib.ctypes.c_int64 * 3)(*k_cache.stride()[:3]),
-            slot_mapping.data_ptr(), k_cache.shape[2], _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv),
+            slot_mapping.data_ptr(), k_cache.shape[2], _lib.ptr(pk), _lib.ptr(pv), _lib.ptr(dq),
+            _lib.ptr(dk), _lib.ptr(dv),
             T, n_tok, num_q_heads, num_kv_heads, head_dim, _lib.stream_of(dev),
         ),
         "qkv_rope_lif_pack",

@@ -211,6 +211,79 @@ def gather_kv_unpacked_pair(
     return _gather(k_cache, v_cache, block_table, seq_len, head_dim, block_size, dtype)
 
 
+PREFILL_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+
+
+def prefill_supported(head_dim: int, dtype: torch.dtype) -> bool:
+    """Whether :func:`paged_spike_attn_prefill` takes these chunks."""
+    return 0 < head_dim <= 128 and dtype in PREFILL_DTYPES
+
+
+def paged_spike_attn_prefill(
+    q_packed: torch.Tensor,
+    k_words: torch.Tensor,
+    v_words: torch.Tensor,
+    chunks: list[tuple[int, int, int, int, torch.Tensor | None]],
+    out: torch.Tensor,
+    head_dim: int,
+    block_size: int,
+) -> torch.Tensor:
+    """Causal attention of prefill chunks on packed spikes, one launch
+    (replaces the unpack-gather + SDPA of spikeinfer/attention.py:161-178).
+
+    ``q_packed`` ``int32 [T, rows, H_q, W]`` and ``out`` ``[T, n_tok, H_q,
+    head_dim]`` (any strides, last axis contiguous); ``k_words``/``v_words``
+    ``int32 [T, H_kv, slots, W]`` of one layout.  Each chunk is ``(q_row,
+    out_row, q_len, ctx, table)``: its queries are rows ``q_row ..`` of
+    ``q_packed``, its outputs rows ``out_row ..`` of ``out``, and key ``j`` of
+    its ``ctx + q_len`` is found through the block-table row ``table``, or,
+    with ``table`` None (``ctx`` 0), in slot ``q_row + j`` of ``k_words``.
+    ``out_row - q_row`` is the same for all chunks.
+    """
+    T, _, n_heads, words = q_packed.shape
+    dev = _lib.require_gpu(q_packed, k_words, v_words, out)
+    for name, t in (("q_packed", q_packed), ("k", k_words), ("v", v_words)):
+        _check_packed(name, t)
+    if words != packed_width(head_dim) or k_words.shape[3] != words or k_words.shape[0] != T:
+        raise ValueError(f"words of {tuple(q_packed.shape)} / {tuple(k_words.shape)} do not fit head_dim={head_dim}")
+    if k_words.shape != v_words.shape or k_words.stride() != v_words.stride():
+        raise ValueError("k and v caches must have the same shape and strides")
+    if out.ndim != 4 or out.shape[0] != T or tuple(out.shape[2:]) != (n_heads, head_dim) or out.stride(-1) != 1:
+        raise ValueError(f"out must be [{T}, n_tok, {n_heads}, {head_dim}] with contiguous channels")
+    packed, keep, shift = [], [], None
+    for q_row, out_row, q_len, ctx, table in chunks:
+        if q_len <= 0:
+            continue
+        if q_row < 0 or q_row + q_len > q_packed.shape[1] or out_row < 0 or out_row + q_len > out.shape[1]:
+            raise ValueError(f"chunk rows {q_row}, {out_row} + {q_len} outside q or out")
+        if shift is None:
+            shift = out_row - q_row
+        elif shift != out_row - q_row:
+            raise ValueError("every chunk needs the same offset between its q and out rows")
+        if table is None:
+            packed.append(_lib.pack_prefill_chunk(q_row, 0, 0, 0, q_len, ctx))
+            continue
+        _lib.require_gpu(q_packed, table)
+        table = _as_int32(table)
+        if table.ndim != 1:
+            raise ValueError("block_table must be one sequence's 1-D row")
+        keep.append(table)
+        packed.append(_lib.pack_prefill_chunk(q_row, table.data_ptr(), table.stride(0), table.numel(), q_len, ctx))
+    if not packed:
+        return out
+    esz = out.element_size()
+    _lib.check(
+        _lib.load().spk_prefill_attn(
+            q_packed.data_ptr(), _lib.strides(q_packed), k_words.data_ptr(), v_words.data_ptr(),
+            _lib.strides(k_words), k_words.shape[2], b"".join(packed), len(packed),
+            out.data_ptr() + shift * out.stride(1) * esz, _lib.dtype_code(out.dtype), _lib.strides(out), T,
+            n_heads, k_words.shape[1], head_dim, block_size, 1.0 / math.sqrt(head_dim), _lib.stream_of(dev),
+        ),
+        "paged_spike_attn_prefill",
+    )
+    return out
+
+
 def paged_spike_attn_decode_partials(
     q_packed: torch.Tensor,
     k_cache: torch.Tensor,

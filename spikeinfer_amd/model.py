@@ -37,7 +37,8 @@ from .kernels.decoder_ops import (add_rmsnorm, embed_rmsnorm, lif_gate_mul, line
                                   mlp_gate_lif, norm_linear_decode, norm_mlp_gate_lif, pack_gate_up,
                                   pack_linear, qkv_decode_attention, qkv_rope_lif_pack, rmsnorm_mean_t)
 from .kernels.packing import packed_width
-from .kernels.spike_attention import gather_kv_unpacked_pair, paged_spike_attn_decode
+from .kernels.spike_attention import (gather_kv_unpacked_pair, paged_spike_attn_decode,
+                                      paged_spike_attn_prefill, prefill_supported)
 
 
 @dataclass
@@ -228,14 +229,22 @@ class SpikingDecoder:
         bufs = bufs or {}
         positions = positions.to(torch.int64).contiguous()
         h, x = embed_rmsnorm(input_ids, self.embed, self.layers[0].input_norm, c.rms_norm_eps, T)
+        # Prefill chunks attend on packed words; dense spikes (SDPA) only for
+        # head dims the packed kernel does not take.
+        packed_prefill = bool(meta.num_prefills) and prefill_supported(D, self.dtype)
+        n_q = n if packed_prefill else n_dec
         q_packed = bufs.get("q_packed")
-        if n_dec and q_packed is None:
-            q_packed = torch.empty((T, n_dec, Hq, self.W), dtype=torch.int32, device=h.device)
+        if n_q and (q_packed is None or packed_prefill):
+            q_packed = torch.empty((T, n_q, Hq, self.W), dtype=torch.int32, device=h.device)
+        kv_packed = None
+        if packed_prefill and 0 in meta.prefill_context_lens:
+            kv_packed = tuple(torch.empty((T, n, Hkv, self.W), dtype=torch.int32, device=h.device)
+                              for _ in range(2))
         attn = bufs.get("attn")
         if attn is None:
             attn = torch.empty((T, n, Hq, D), dtype=self.dtype, device=h.device)
         dense = None
-        if meta.num_prefills:
+        if meta.num_prefills and not packed_prefill:
             dense = (torch.empty((T, Hq, n, D), dtype=self.dtype, device=h.device),
                      torch.empty((T, Hkv, n, D), dtype=self.dtype, device=h.device),
                      torch.empty((T, Hkv, n, D), dtype=self.dtype, device=h.device))
@@ -263,12 +272,14 @@ class SpikingDecoder:
             if not fused:
                 qkv_rope_lif_pack(qkv, self.rope_cos, self.rope_sin, L.lif_qkv_beta, L.lif_qkv_th,
                                   k_cache, v_cache, meta.slot_mapping, Hq, Hkv, D, q_packed=q_packed,
-                                  n_q=n_dec, dense=dense, positions=positions)
+                                  n_q=n_q, dense=dense, positions=positions, kv_packed=kv_packed)
             if n_dec and not fused:
-                paged_spike_attn_decode(q_packed, k_cache, v_cache, meta.block_tables, meta.seq_lens,
+                paged_spike_attn_decode(q_packed[:, :n_dec], k_cache, v_cache, meta.block_tables, meta.seq_lens,
                                         head_dim=D, block_size=meta.block_size, num_q_heads=Hq,
                                         num_kv_heads=Hkv, out=attn[:, :n_dec])
-            if meta.num_prefills:
+            if packed_prefill:
+                self._packed_prefill_attention(q_packed, kv_packed, k_cache, v_cache, meta, attn)
+            elif meta.num_prefills:
                 self._prefill_attention(dense, k_cache, v_cache, meta, attn)
             o = self._linear(attn.view(T, n, Hq * D), L.w_o, None, L.w_o_packed, n)
             y = None
@@ -289,6 +300,24 @@ class SpikingDecoder:
             if delta is None:
                 delta = F.linear(y, L.w_down)
         return rmsnorm_mean_t(h, self.final_norm, c.rms_norm_eps, delta=delta)
+
+    def _packed_prefill_attention(self, q_packed, kv_packed, k_cache, v_cache, meta: AttentionMetadata,
+                                  attn) -> None:
+        """Prefill chunks (attention.py:161-178) on packed words: a chunk with a
+        cached prefix reads its keys through its block table, one without
+        attends to the words its own tokens just produced."""
+        fresh, cached = [], []
+        for start, q_len, ctx, table in zip(meta.prefill_query_starts, meta.prefill_query_lens,
+                                            meta.prefill_context_lens, meta.prefill_block_tables):
+            if ctx == 0:
+                fresh.append((start, start, q_len, 0, None))
+            else:
+                cached.append((start, start, q_len, ctx, table))
+        if fresh:
+            k, v = (w.permute(0, 2, 1, 3) for w in kv_packed)
+            paged_spike_attn_prefill(q_packed, k, v, fresh, attn, self.D, meta.block_size)
+        if cached:
+            paged_spike_attn_prefill(q_packed, k_cache, v_cache, cached, attn, self.D, meta.block_size)
 
     def _prefill_attention(self, dense, k_cache, v_cache, meta: AttentionMetadata, attn) -> None:
         """Prefill chunks (attention.py:161-178): SDPA on the chunk's dense
