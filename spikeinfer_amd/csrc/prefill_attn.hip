@@ -13,8 +13,11 @@
 //     32-key tiles round-robin and add their sums at the end in wave order, so a
 //     row's sums depend on its own sequence only, never on the batch or on QT.
 //   * Scores: S^T[key, row] = K Q^T as one v_mfma_scale_f32_32x32x64_f8f6f4 per
-//     64 channels, bits as fp4 0.5 (bit i of nibble group i in place), block scale
-//     2^4: the accumulators are exactly 4 * popc(q & k).
+//     64 channels, bits as fp4 0.5 (bit i of nibble group i in place), block scales
+//     2^-72 and 2^-73: an accumulator is the subnormal 4 * popc(q & k) * 2^-149, so
+//     its bits are the integer 4 * popc(q & k) and need no conversion (the matrix
+//     cores keep subnormals; 16 conversions a tile: 145 -> 138 us on the prompt
+//     below).
 //   * A score is an integer in 0..head_dim, so its weight exp(score * scale) is a
 //     table entry at byte 4 * score: (hi, lo) halves of an f16 pair with hi + lo
 //     the weight to 2^-23 (the table spans e^sqrt(head_dim) <= 2^17 below 2^15, so
@@ -27,10 +30,17 @@
 //     is an operand register as it is.  V^T comes from a 32 x 32 bit transpose of
 //     the wave's V words (five lane-exchange steps), each bit as the pair 1.0, 1.0;
 //     it is built once per key tile and shared by the QT row tiles.
-//   * Denominators: v_dot2_f32_f16 of the pair with (1, 1) into fp32.
-// What bounds it: the matrix cores (two f16 products per weight keep it at 32-bit
-// precision: 256 of ~290 cycles per 32 x 32 tile at head_dim 64), the lookups and
-// conversions fill the VALU and LDS beside them.
+//   * Denominators: v_dot2_f32_f16 of the pair with (1, 1), 16 weights to a
+//     partial sum and the partial sums in fp32 (one long dot2 chain per row lost
+//     1e-6 at 4,000 keys).  Error against float64, fp32 output: 4.1e-7 at 4,000
+//     keys, 4.6e-7 at 16,000; fp32 SDPA 7.9e-7 and 1.3e-5.
+// What bounds it: issue.  A 32 x 32 tile at head_dim 64 takes 288 cycles of matrix
+// core (two f16 products a weight keep it at 32-bit precision) and about 330 of
+// VALU, and the two overlap little: 720 measured (a 4,096-token prompt, 14 / 2
+// heads, T = 4: 135 us; row tiles one after the other, without the next one's
+// lookups under this one's products: 175).  Against unpack + SDPA (one layer, LIF
+// included, bf16): that prompt 8,693 -> 142 us; 32 decodes with chunks of 509 and
+// 472 behind 1,024 and 923 cached tokens 1,035 -> 59 us.
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -56,9 +66,10 @@ constexpr int kTab = 129;       // weights of scores 0..head_dim (<= 128)
 
 struct Chunk {
   int64_t start;         // first batch row
-  const int32_t *table;  // block-table row, or nullptr: key j is slot start + j
+  const int32_t *table;  // block-table row (any readable word when direct)
   int64_t tstride;
   int n_table, q_len, ctx;
+  int direct;            // key j is slot start + j, no table
   int tile0;             // first row tile of the chunk in the launch
 };
 
@@ -71,6 +82,7 @@ struct Params {
   void *out;                   // (t, batch row, query head, channel)
   int64_t os0, os1, os2;
   int out_dtype, out_vec;      // out_vec: rows take aligned 4-channel stores
+  uint32_t rep_mul;            // floor(r / nrep) = r * rep_mul >> 32 for every row
   int units, Hkv, nrep, D, W, bs_log2, nchunks;
   uint32_t tab[kTab];
   Chunk c[kMaxChunks];
@@ -147,6 +159,9 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
   const int ntile = (rows + 32 * QT - 1) / (32 * QT);
   const int r0 = (ntile - 1 - (tile - p.c[ci].tile0)) * 32 * QT;  // longest tiles first
   const int nq = min(QT, (rows - r0 + 31) >> 5);
+  auto token_of = [&](int r) {
+    return p.nrep == 1 ? r : static_cast<int>(__umulhi(static_cast<uint32_t>(r), p.rep_mul));
+  };
 
   if (tid <= p.D) tab[tid] = p.tab[tid];
 
@@ -158,10 +173,10 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
   for (int i = 0; i < QT; ++i) {
     const int r = min(r0 + 32 * i + col, rows - 1);
-    const int tok = r / p.nrep, h = r - tok * p.nrep;
+    const int tok = token_of(r), h = r - tok * p.nrep;
     lim[i] = ctx + tok;
-    lo[i] = ctx + min(r0 + 32 * i, rows - 1) / p.nrep;
-    hi[i] = ctx + min(r0 + 32 * i + 31, rows - 1) / p.nrep;
+    lo[i] = ctx + token_of(min(r0 + 32 * i, rows - 1));
+    hi[i] = ctx + token_of(min(r0 + 32 * i + 31, rows - 1));
     const uint32_t *qp = p.q + t * p.qs0 + (start + tok) * p.qs1 + (kvh * p.nrep + h) * p.qs2;
 #pragma unroll
     for (int s = 0; s < NK; ++s) {
@@ -173,30 +188,32 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
   const int32_t *table = p.c[ci].table;
   const int64_t tstride = p.c[ci].tstride;
   const int n_table = p.c[ci].n_table;
+  const bool direct = p.c[ci].direct;
   const int kv_len = ctx + q_len;
   const int bs_mask = (1 << p.bs_log2) - 1;
   const uint32_t nblocks = static_cast<uint32_t>(min<int64_t>(p.num_slots >> p.bs_log2, 0xffffffffll));
   const uint32_t *kbase = p.k + t * p.ks0 + kvh * p.ks1;
   const uint32_t *vbase = p.v + t * p.ks0 + kvh * p.ks1;
-  // Slot of key j, -1 where the sequence or its table has none (zero spikes).
-  auto slot_of = [&](int kt) -> int64_t {
-    const int j = kt * kKeys + col;
-    if (j >= kv_len) return -1;
-    if (!table) return start + j;
-    const int blk = j >> p.bs_log2;
-    if (blk >= n_table) return -1;
-    const uint32_t phys = static_cast<uint32_t>(table[blk * tstride]);
-    return phys < nblocks ? (static_cast<int64_t>(phys) << p.bs_log2) | (j & bs_mask) : -1;
+  // Loads are unconditional (indices clamped into range, the value dropped where
+  // the sequence, its table or the cache ends: zero spikes), so that the wave
+  // waits for none of them before it is used an iteration later.
+  auto block_of = [&](int kt) -> uint32_t {
+    const int blk = (kt * kKeys + col) >> p.bs_log2;
+    return static_cast<uint32_t>(table[min(blk, n_table - 1) * tstride]);
   };
-  auto load = [&](int64_t slot, uint32_t (&kw)[NK], uint32_t (&vw)[NK]) {
+  auto load = [&](int kt, uint32_t phys, uint32_t (&kw)[NK], uint32_t (&vw)[NK], bool &ok) {
+    const int j = kt * kKeys + col;
+    ok = j < kv_len && (direct || ((j >> p.bs_log2) < n_table && phys < nblocks));
+    const int64_t slot = direct ? start + j : (static_cast<int64_t>(phys) << p.bs_log2) | (j & bs_mask);
+    const int64_t at = ok ? slot * p.ks2 : (direct ? start * p.ks2 : 0);
 #pragma unroll
     for (int s = 0; s < NK; ++s) {
-      const int w = 2 * s + half;
-      const bool ok = slot >= 0 && w < p.W;
-      kw[s] = ok ? kbase[slot * p.ks2 + w] : 0u;
-      vw[s] = ok ? vbase[slot * p.ks2 + w] : 0u;
+      const int w = min(2 * s + half, p.W - 1);
+      kw[s] = kbase[at + w];
+      vw[s] = vbase[at + w];
     }
   };
+  auto keep = [&](uint32_t x, int s, bool ok) { return ok && 2 * s + half < p.W ? x : 0u; };
 
   v16f acc[QT][NC];
   float l[QT];
@@ -208,27 +225,28 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
   }
   __syncthreads();
 
-  const int nkt = (ctx + min(r0 + 32 * nq - 1, rows - 1) / p.nrep) / kKeys + 1;
+  const int nkt = (ctx + token_of(min(r0 + 32 * nq - 1, rows - 1))) / kKeys + 1;
   uint32_t kw[NK], vw[NK];
-  load(slot_of(wave), kw, vw);
-  int64_t snext = slot_of(wave + kWaves);
+  bool ok;
+  load(wave, block_of(wave), kw, vw, ok);
+  uint32_t pnext = block_of(wave + kWaves);
   for (int kt = wave; kt < nkt; kt += kWaves) {
-    // Operands of this tile; the next tile's words and the slots of the one
+    // Operands of this tile; the next tile's words and the block of the one
     // after are requested before they are used.
     v8i kop[NK];
     uint32_t vt[2 * NK];
 #pragma unroll
     for (int s = 0; s < NK; ++s) {
-      kop[s] = fp4_bits(kw[s]);
-      const uint32_t x = transpose32(vw[s], lane);
+      kop[s] = fp4_bits(keep(kw[s], s, ok));
+      const uint32_t x = transpose32(keep(vw[s], s, ok), lane);
       // Both halves of the wave need every channel tile: lanes l and l + 32 take
       // keys 4 * (l / 32) + 0..3 of each eight.
       const auto sw = __builtin_amdgcn_permlane32_swap(x, x, false, false);
       vt[2 * s] = sw[0] >> (4 * half);
       vt[2 * s + 1] = sw[1] >> (4 * half);
     }
-    load(snext, kw, vw);
-    snext = slot_of(kt + 2 * kWaves);
+    load(kt + kWaves, pnext, kw, vw, ok);
+    pnext = block_of(kt + 2 * kWaves);
     v8h vop[NC][4];
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -240,36 +258,59 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
           x[i] = static_cast<uint32_t>(static_cast<int>(vt[c] << (31 - 8 * g - i)) >> 31) & 0x3c003c00u;
         vop[c][g] = __builtin_bit_cast(v8h, x);
       }
-    auto row_tile = [&](int i, auto masked) {
+    auto scores = [&](int i) {
       v16f s = {};
 #pragma unroll
       for (int k = 0; k < NK; ++k)
-        s = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kop[k], qop[i][k], s, 4, 4, 0, 131, 0, 127);
+        s = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kop[k], qop[i][k], s, 4, 4, 0, 55, 0, 54);
+      return s;
+    };
+    auto lookup = [&](const v16f &s, uint32_t (&w)[16]) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const uint32_t at = tab0 + __float_as_uint(s[e]);
+        w[e] = *reinterpret_cast<const SPK_LDS uint32_t *>(static_cast<uintptr_t>(at));
+      }
+    };
+    auto products = [&](int i, const uint32_t (&w)[16], auto masked) {
+      float d[4] = {0.f, 0.f, 0.f, 0.f};  // (a chain of dot2 on one register waits for itself)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        v4u w;
+        v4u x;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const uint32_t at = static_cast<uint32_t>(s[4 * g + e]);
-          uint32_t x = *reinterpret_cast<const SPK_LDS uint32_t *>(static_cast<uintptr_t>(tab0 + at));
-          if constexpr (decltype(masked)::value) x = kt * kKeys + 8 * g + 4 * half + e <= lim[i] ? x : 0u;
-          w[e] = x;
-          l[i] = __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, x), v2h{1, 1}, l[i], false);
+          uint32_t y = w[4 * g + e];
+          if constexpr (decltype(masked)::value) y = kt * kKeys + 8 * g + 4 * half + e <= lim[i] ? y : 0u;
+          d[e] = __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, y), v2h{1, 1}, d[e], false);
+          x[e] = y;
         }
-        const v8h pw = __builtin_bit_cast(v8h, w);
+        const v8h pw = __builtin_bit_cast(v8h, x);
 #pragma unroll
         for (int c = 0; c < NC; ++c)
           acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vop[c][g], pw, acc[i][c], 0, 0, 0);
       }
+      l[i] += (d[0] + d[1]) + (d[2] + d[3]);
     };
     if (nq == QT && kt * kKeys + kKeys - 1 <= lo[0]) {
+      // The next row tile's scores are computed and looked up under this one's
+      // products.
+      uint32_t w[2][16];
+      lookup(scores(0), w[0]);
 #pragma unroll
-      for (int i = 0; i < QT; ++i) row_tile(i, std::false_type{});
+      for (int i = 0; i < QT; ++i) {
+        if (i + 1 < QT) lookup(scores(i + 1), w[(i + 1) & 1]);
+        products(i, w[i & 1], std::false_type{});
+        // Row tile by row tile: left free, the scheduler hoists lookups of several
+        // and spills (head_dim 128: 198 us instead of 77).
+        __builtin_amdgcn_sched_barrier(0);
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < QT; ++i) {
         if (i >= nq || kt * kKeys > hi[i]) continue;
-        row_tile(i, std::true_type{});
+        uint32_t w[16];
+        lookup(scores(i), w);
+        products(i, w, std::true_type{});
       }
     }
   }
@@ -299,39 +340,45 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
     float den = 0.f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) den += lsum[i][w][col] + lsum[i][w][col + 32];
-    const int tok = r / p.nrep, h = r - tok * p.nrep;
+    const float inv = 1.f / den;
+    const int tok = token_of(r), h = r - tok * p.nrep;
     const int64_t row = t * p.os0 + (start + tok) * p.os1 + (kvh * p.nrep + h) * p.os2;
+    auto value = [&](int j) {
+      float a = 0.f;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float o[4];
+      for (int w = 0; w < kWaves; ++w) a += red[wave][w][j][lane];
+      return a * inv;
+    };
+    if (p.out_vec) {  // D % 4 == 0: four channels lie in or out together
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float a = 0.f;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) a += red[wave][w][4 * g + e][lane];
-        o[e] = a / den;
-      }
-      const int ch = 32 * c + 8 * g + 4 * half;
-      if (p.out_vec) {  // D % 4 == 0: the four channels lie in or out together
+      for (int g = 0; g < 4; ++g) {
+        const int ch = 32 * c + 8 * g + 4 * half;
+        const float o[4] = {value(4 * g), value(4 * g + 1), value(4 * g + 2), value(4 * g + 3)};
         if (ch >= p.D) continue;
         if (p.out_dtype == SPK_F32) {
           *reinterpret_cast<v4f *>(static_cast<float *>(p.out) + row + ch) = v4f{o[0], o[1], o[2], o[3]};
-        } else {
-          uint32_t w2[2];
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const bool b = p.out_dtype == SPK_BF16;
-            const uint32_t x0 = b ? f32_to_bf16_bits(o[2 * e]) : __builtin_bit_cast(uint16_t, static_cast<_Float16>(o[2 * e]));
-            const uint32_t x1 = b ? f32_to_bf16_bits(o[2 * e + 1])
-                                  : __builtin_bit_cast(uint16_t, static_cast<_Float16>(o[2 * e + 1]));
-            w2[e] = x0 | (x1 << 16);
-          }
-          *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(p.out) + row + ch) = make_uint2(w2[0], w2[1]);
+          continue;
         }
-      } else {
+        uint32_t w2[2];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (ch + e < p.D) store_f32_as(p.out, row + ch + e, p.out_dtype, o[e]);
+        for (int e = 0; e < 2; ++e) {
+          uint16_t x0, x1;
+          if (p.out_dtype == SPK_BF16) {
+            x0 = f32_to_bf16_bits(o[2 * e]);
+            x1 = f32_to_bf16_bits(o[2 * e + 1]);
+          } else {
+            x0 = __builtin_bit_cast(uint16_t, static_cast<_Float16>(o[2 * e]));
+            x1 = __builtin_bit_cast(uint16_t, static_cast<_Float16>(o[2 * e + 1]));
+          }
+          w2[e] = x0 | (static_cast<uint32_t>(x1) << 16);
+        }
+        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(p.out) + row + ch) = make_uint2(w2[0], w2[1]);
+      }
+    } else {
+#pragma unroll 1
+      for (int j = 0; j < 16; ++j) {
+        const int ch = 32 * c + 8 * (j >> 2) + 4 * half + (j & 3);
+        if (ch < p.D) store_f32_as(p.out, row + ch, p.out_dtype, value(j));
       }
     }
   }
@@ -364,7 +411,7 @@ static void launch(const Params &p, unsigned grid, hipStream_t s) {
     case 1: prefill_attn_kernel<QT, 1><<<grid, kWaves * 64, 0, s>>>(p); break;
     case 2: prefill_attn_kernel<QT, 2><<<grid, kWaves * 64, 0, s>>>(p); break;
     case 3: prefill_attn_kernel<QT < 2 ? QT : 2, 3><<<grid, kWaves * 64, 0, s>>>(p); break;
-    default: prefill_attn_kernel<QT < 2 ? QT : 2, 4><<<grid, kWaves * 64, 0, s>>>(p); break;
+    default: prefill_attn_kernel<1, 4><<<grid, kWaves * 64, 0, s>>>(p); break;
   }
 }
 
@@ -386,14 +433,15 @@ extern "C" int spk_prefill_attn(const int32_t *q, const int64_t q_strides[3], co
   if (!(scale > 0.f) || scale * head_dim > 12.f)  // the table's span within f16
     return fail(SPK_EINVAL, "prefill_attn: scale=%g outside (0, 12/head_dim]", (double)scale);
   if (nchunks == 0) return SPK_OK;
-  if (!q || !k || !v || !out || !chunks) return fail(SPK_EINVAL, "prefill_attn: null pointer");
+  if (!q || !out || !chunks || (num_slots > 0 && (!k || !v))) return fail(SPK_EINVAL, "prefill_attn: null pointer");
   const int nrep = Hq / Hkv;
   int64_t total = 0;  // rows of all chunks
   for (int i = 0; i < nchunks; ++i) {
     const SpkPrefillChunk &c = chunks[i];
     if (c.start < 0 || c.q_len < 0 || c.ctx < 0 || c.n_table < 0 || (!c.table && c.ctx != 0))
       return fail(SPK_EINVAL, "prefill_attn: chunk %d: start=%lld q_len=%d ctx=%d", i, (long long)c.start, c.q_len, c.ctx);
-    if (static_cast<int64_t>(c.q_len) * nrep > (1 << 28) || static_cast<int64_t>(c.q_len) + c.ctx > (1 << 30))
+    const int64_t rows = static_cast<int64_t>(c.q_len) * nrep;
+    if (rows > (1 << 28) || rows * nrep > 0xffffffffll || static_cast<int64_t>(c.q_len) + c.ctx > (1 << 30))
       return fail(SPK_EUNSUPPORTED, "prefill_attn: chunk %d of %d + %d tokens is too long", i, c.ctx, c.q_len);
     if (!c.table && c.start + c.q_len > num_slots)
       return fail(SPK_EINVAL, "prefill_attn: chunk %d reaches past %lld slots", i, (long long)num_slots);
@@ -406,18 +454,26 @@ extern "C" int spk_prefill_attn(const int32_t *q, const int64_t q_strides[3], co
   p.v = reinterpret_cast<const uint32_t *>(v);
   p.ks0 = kv_strides[0]; p.ks1 = kv_strides[1]; p.ks2 = kv_strides[2];
   p.num_slots = num_slots;
+  if (num_slots <= 0) {  // an empty cache: every key is dropped, the loads read q's first words
+    p.k = p.v = p.q;
+    p.ks0 = p.ks1 = p.ks2 = 0;
+  }
   p.out = out; p.out_dtype = out_dtype;
   p.os0 = out_strides[0]; p.os1 = out_strides[1]; p.os2 = out_strides[2];
   p.out_vec = head_dim % 4 == 0 && p.os0 % 4 == 0 && p.os1 % 4 == 0 && p.os2 % 4 == 0 &&
               (reinterpret_cast<uintptr_t>(out) & 15) == 0;
   p.units = T * Hkv; p.Hkv = Hkv; p.nrep = nrep; p.D = head_dim; p.W = (head_dim + 31) / 32;
   p.bs_log2 = ilog2(block_size);
+  // ceil(2^32 / nrep): its product with r is off by less than r * nrep <= 2^32
+  p.rep_mul = static_cast<uint32_t>(((int64_t(1) << 32) + nrep - 1) / nrep);
   prefill::build_table(scale, head_dim, p.tab);
   // Row tiles per workgroup: four share a key tile's V operands; fewer while
-  // that leaves under two workgroups a CU.  The sums do not depend on it.
+  // that leaves under two workgroups a CU, and where their sums would not fit
+  // the registers (head_dim 128, 2,000 tokens: one 60 us, two 77).  The sums do
+  // not depend on it.
   const int64_t tiles = (total + 31) / 32 * p.units;
   const int qt = tiles >= 4 * 512 ? 4 : (tiles >= 2 * 512 ? 2 : 1);
-  const int qt_used = head_dim > 64 && qt > 2 ? 2 : qt;
+  const int qt_used = head_dim > 96 ? 1 : (head_dim > 64 && qt > 2 ? 2 : qt);
   hipStream_t s = static_cast<hipStream_t>(stream);
   for (int i = 0; i < nchunks;) {
     int64_t grid = 0;
@@ -430,7 +486,11 @@ extern "C" int spk_prefill_attn(const int32_t *q, const int64_t q_strides[3], co
         if (p.nchunks) break;
         return fail(SPK_EUNSUPPORTED, "prefill_attn: chunk %d is too large for one launch", i);
       }
-      p.c[p.nchunks++] = prefill::Chunk{c.start, c.table, c.table_stride, c.n_table, c.q_len, c.ctx,
+      // The kernel loads a table entry whether it uses it or not: a direct chunk
+      // or an empty table gets a readable word.
+      const bool none = !c.table || c.n_table == 0;
+      p.c[p.nchunks++] = prefill::Chunk{c.start, none ? q : c.table, none ? 0 : c.table_stride,
+                                        c.table ? c.n_table : 0, c.q_len, c.ctx, c.table ? 0 : 1,
                                         static_cast<int>(grid)};
       grid += nt;
     }
