@@ -490,16 +490,21 @@ __device__ __forceinline__ int64_t filter_and_draw(const Src src, Shared &sh, co
 // rows with 0 < top_k <= kFastMaxK a first launch splits each row into
 // kSlices slices, one workgroup each (sample_slices_kernel):
 //   * the slice goes into registers once, with the penalties, as keys of the
-//     penalised values v; every kSampleStride-th one is a sample;
-//   * the r-th largest sample (r = k / kSampleStride + 3, doubled while the
-//     candidates fall short) fixes a bound x_B on x = v / temperature, turned
-//     once into the smallest v key whose x reaches x_B (a bisection over keys,
-//     x monotone in v), so the passes compare keys and divide only the
-//     candidates {x >= x_B}, a prefix of the slice in the total order (x
-//     descending, index ascending);
-//   * with at least k of them (or the whole slice) they hold the slice's k
-//     largest: each candidate's rank among them is counted, and the first
-//     min(k, n) go to the workspace in order.
+//     penalised values v, and each thread keeps its largest;
+//   * a value that at least k of the threads' largest reach has at least k
+//     elements at or above it, and few more: of n random values over 512
+//     threads about -512 ln(1 - k / 512), 53 for k = 50.  A bisection on the 512
+//     maxima finds one; it fixes a bound x_B on x = v / temperature, turned
+//     once into the smallest v key whose x reaches x_B (x is monotone in v),
+//     so the pass that gathers the candidates {x >= x_B}, a prefix of the slice
+//     in the total order (x descending, index ascending), compares keys and
+//     divides only those;
+//   * they hold the slice's k largest: each candidate's rank among them is
+//     counted, and the first min(k, n) go to the workspace in order.
+// What bounds it: VALU over the slice's elements and the phases between
+// barriers; 64 rows of 151,936 bf16 logits, top-k 50: 13 us (with a bound
+// from every 32nd element, about 160 candidates a slice, and the registers of
+// the largest vocabulary: 30), the row kernel 11 (13 with its round trips in a row).
 // The row kernel then merges a row's lists (ranks by binary search), which
 // gives the row's top-k in order, and finishes with prefix sums over it:
 // min_p, top_p and the draw are the same cuts as filter_and_draw's, computed
@@ -512,8 +517,6 @@ constexpr int kSliceCand = 1024;
 constexpr int kFastMaxK = 256;
 static_assert(kFastMaxK < kThreads, "the finish takes one thread per kept position");
 constexpr int kSliceMaxLen = ((kMaxVocab + kSlices - 1) / kSlices + 255) & ~255;
-constexpr int kSliceSamples = kSliceMaxLen / kSampleStride;
-constexpr int kSampleRegs = kSliceSamples / 64;  // samples a lane of wave 0 reads
 
 __host__ __device__ inline int slice_len(int V) { return ((V + kSlices - 1) / kSlices + 255) & ~255; }
 
@@ -599,30 +602,38 @@ struct SliceShared {
   uint32_t seen[kSliceMaxLen / 32];  // the slice's generated-token bits
   int32_t hkey[kHashSlots];          // token + 1 -> count, tokens of the slice
   int32_t hcnt[kHashSlots];
-  uint32_t samp[kSliceSamples];      // sample keys (of v)
+  uint32_t tmax[kSliceThreads];      // key of each thread's largest v, 0 without elements
   unsigned long long cand[kSliceCand + 16];  // candidates' order keys (+ a zero batch)
   float fmax[kSliceThreads / 64];
-  uint32_t wcount[kSliceThreads / 64];
   unsigned long long zw[kSliceThreads / 64];
-  uint32_t bound;
+  uint32_t bound, count;
 };
 
 // A thread's share of a slice: vectors v = threadIdx.x + q * kSliceThreads
-// of the slice's whole vectors (elements v * W ..), every load issued at once
-// (vectors past them re-read the first and are dropped), plus one of the < W
-// trailing elements.  After pass A it holds the keys of the penalised
-// logits, so later passes only compare keys.  No load leaves the slice.
-// Needs 16-byte aligned rows (the host checks).
-template <int DT>
+// of the slice's whole vectors (elements v * W ..), q < NQ, every load issued at
+// once, plus one of the < W trailing elements and the generated tokens it was
+// the first to mark (kOwn at most).  Slots hold keys of the penalised logits:
+// q * W + j, then the trailing element, then the owned tokens; an element that
+// is owned as a token, or does not exist, has key 0 in its own slot, so every
+// element counts once.  No load leaves the slice.  Needs 16-byte aligned rows
+// (the host checks).
+//
+// The code is kept short -- no per-element penalty, the gathering pass loops
+// over the few slots that reach the bound -- because a workgroup runs it once
+// and waits for its instructions: unrolled over the slots it took 23 KB.
+template <int DT, int NQ>
 struct SliceRegs {
   typedef typename Elem<DT>::T E;
   static constexpr int W = Elem<DT>::kVec;
-  static constexpr int kVecs = kSliceMaxLen / (W * kSliceThreads);
+  static constexpr int kOwn = kMaxHist / kSliceThreads;
+  static constexpr int kTail = NQ * W;
+  static constexpr int kSlots = kTail + 1 + kOwn;
   typedef E Vec __attribute__((ext_vector_type(W)));
-  Vec a[kVecs];
+  Vec a[NQ];
   E tail;
-  uint32_t key[kVecs * W + 1];  // slot q * W + j; the last one the trailing element
-  int nv;                       // whole vectors of the slice
+  uint32_t key[kSlots];
+  int32_t own[kOwn];  // owned tokens (offset in the slice), -1: none
+  int nv;             // whole vectors of the slice
   bool tail_valid;
 
   __device__ __forceinline__ void load(const E *row, int c0, int n) {
@@ -630,7 +641,7 @@ struct SliceRegs {
     nv = n / W;
     if (nv > 0) {  // (a slice of fewer than W elements has no whole vector to re-read)
 #pragma unroll
-      for (int q = 0; q < kVecs; ++q) {
+      for (int q = 0; q < NQ; ++q) {
         const int v = threadIdx.x + q * kSliceThreads;
         a[q] = pv[v < nv ? v : 0];
       }
@@ -638,40 +649,62 @@ struct SliceRegs {
     const int t = nv * W + static_cast<int>(threadIdx.x);
     tail_valid = t < n;
     tail = row[c0 + (tail_valid ? t : 0)];
-  }
-  __device__ __forceinline__ bool valid(int slot) const {
-    return slot == kVecs * W ? tail_valid : static_cast<int>(threadIdx.x) + (slot / W) * kSliceThreads < nv;
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o) own[o] = -1;
   }
   __device__ __forceinline__ int elem(int slot) const {  // offset in the slice
-    return slot == kVecs * W ? nv * W + static_cast<int>(threadIdx.x)
-                             : (static_cast<int>(threadIdx.x) + (slot / W) * kSliceThreads) * W + slot % W;
-  }
-  // Pass A: key of every penalised logit; f(b, v) for each valid element.
-  template <class F>
-  __device__ __forceinline__ void penalise_all(int c0, const Params &P, const SliceShared &sh, bool has_hist, F f) {
+    if (slot < kTail) return (static_cast<int>(threadIdx.x) + (slot / W) * kSliceThreads) * W + slot % W;
+    int e = nv * W + static_cast<int>(threadIdx.x);
 #pragma unroll
-    for (int q = 0; q < kVecs; ++q) {
-      const int v = threadIdx.x + q * kSliceThreads;
-      const int b = v * W;
-      const bool ok = v < nv;
-      const uint32_t bits = has_hist && ok ? ((sh.seen[b >> 5] >> (b & 31)) & ((1u << W) - 1u)) : 0u;
+    for (int o = 0; o < kOwn; ++o) e = slot == kTail + 1 + o ? own[o] : e;
+    return e;
+  }
+  // Pass A: every slot's key; returns the thread's largest value (NaN aside).
+  __device__ __forceinline__ float fill(const E *row, int c0, const Params &P, const SliceShared &sh, bool has_hist) {
+    float mv = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int b = (static_cast<int>(threadIdx.x) + q * kSliceThreads) * W;
+      uint32_t bits = (1u << W) - 1u;  // elements not counted here
+      if (b < nv * W) bits = has_hist ? (sh.seen[b >> 5] >> (b & 31)) & bits : 0u;
+      float x[W];
 #pragma unroll
       for (int j = 0; j < W; ++j) {
-        float x = elem_to_f32<DT>(a[q][j]);
-        if ((bits >> j) & 1u) x = penalise_seen(P, sh, c0 + b + j, x);
-        key[q * W + j] = fkey(x);
-        if (ok) f(b + j, x);
+        const E e = a[q][j];
+        x[j] = elem_to_f32<DT>(e);
+        key[q * W + j] = fkey(x[j]);
       }
+      if (bits) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+          x[j] = (bits >> j) & 1u ? -INFINITY : x[j];
+          key[q * W + j] = (bits >> j) & 1u ? 0u : key[q * W + j];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < W; ++j) mv = fmaxf(mv, x[j]);
     }
     const int b = nv * W + static_cast<int>(threadIdx.x);
-    float x = elem_to_f32<DT>(tail);
-    if (tail_valid && has_hist && ((sh.seen[b >> 5] >> (b & 31)) & 1u)) x = penalise_seen(P, sh, c0 + b, x);
-    key[kVecs * W] = fkey(x);
-    if (tail_valid) f(b, x);
+    const bool here = tail_valid && !(has_hist && ((sh.seen[b >> 5] >> (b & 31)) & 1u));
+    const float x = here ? elem_to_f32<DT>(tail) : -INFINITY;
+    key[kTail] = here ? fkey(x) : 0u;
+    mv = fmaxf(mv, x);
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o) key[kTail + 1 + o] = 0u;
+    if (has_hist) {
+#pragma unroll
+      for (int o = 0; o < kOwn; ++o) {
+        if (own[o] < 0) continue;
+        const float y = penalise_seen(P, sh, c0 + own[o], elem_to_f32<DT>(row[c0 + own[o]]));
+        key[kTail + 1 + o] = fkey(y);
+        mv = fmaxf(mv, y);
+      }
+    }
+    return mv;
   }
 };
 
-template <int DT, int MODE>
+template <int DT, int MODE, int NQ>
 __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
     const void *logits, int64_t row_stride, int V, const float *temperature, const int32_t *top_k,
     const float *top_p, const float *min_p, const float *rep, const float *presence,
@@ -713,8 +746,9 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
       m_row = fmaxf(m_row, __hip_atomic_load(ws.vmax + static_cast<int64_t>(row) * kSlices + s2,
                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   }
-  SliceRegs<DT> rg;  // the slice's logits, loaded while the history is read
-  rg.load(reinterpret_cast<const E *>(logits) + row * row_stride, c0, c1 - c0);
+  SliceRegs<DT, NQ> rg;  // the slice's logits, loaded while the history is read
+  const E *logits_row = reinterpret_cast<const E *>(logits) + row * row_stride;
+  rg.load(logits_row, c0, c1 - c0);
   // ---- history -> the slice's bits (+ counts) ----
   for (int w = tid; w < (c1 - c0 + 31) / 32; w += kSliceThreads) sh.seen[w] = 0u;
   if (P.use_hash)
@@ -725,11 +759,15 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
     nh = hist_len[row * hist_len_stride];
     const int64_t cap = hist_stride < kMaxHist ? hist_stride : kMaxHist;
     nh = nh < 0 ? 0 : (nh > cap ? static_cast<int>(cap) : nh);
-    for (int j = tid; j < nh; j += kSliceThreads) {
+#pragma unroll
+    for (int o = 0; o < SliceRegs<DT, NQ>::kOwn; ++o) {
+      const int j = tid + o * kSliceThreads;
+      if (j >= nh) break;
       const int64_t tok = history[row * hist_stride + j];
       if (tok < c0 || tok >= c1) continue;
       const int t32 = static_cast<int>(tok);
-      atomicOr(&sh.seen[(t32 - c0) >> 5], 1u << ((t32 - c0) & 31));
+      const uint32_t bit = 1u << ((t32 - c0) & 31);
+      if (!(atomicOr(&sh.seen[(t32 - c0) >> 5], bit) & bit)) rg.own[o] = t32 - c0;  // the first to mark it
       if (P.use_hash) {
         int h = hash_slot(t32);
         while (true) {
@@ -744,12 +782,16 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
   __syncthreads();
   const bool has_hist = nh > 0;
 
-  // ---- maximum and samples (keys of v) ----
-  float mv = -INFINITY;
-  rg.penalise_all(c0, P, sh, has_hist, [&](int b, float v) {
-    mv = fmaxf(mv, v);
-    if (MODE != kModeOpenMax && (b % kSampleStride) == 0) sh.samp[b / kSampleStride] = fkey(v);
-  });
+  // ---- keys and maxima ----
+  constexpr int kSlots = SliceRegs<DT, NQ>::kSlots;
+  float mv = rg.fill(logits_row, c0, P, sh, has_hist);
+  if (MODE != kModeOpenMax) {
+    uint32_t any = 0u;  // (a thread's elements may all be owned by others)
+#pragma unroll
+    for (int q = 0; q < kSlots; ++q) any |= rg.key[q];
+    sh.tmax[tid] = any ? fkey(mv) : 0u;
+    if (tid == 0) sh.count = 0u;
+  }
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) mv = fmaxf(mv, __shfl_xor(mv, d));
   if (lane == 0) sh.fmax[wave] = mv;
@@ -763,86 +805,111 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
     return;
   }
 
-  // ---- bound and candidates.  Wave 0 takes the r-th largest sample, then
-  // the smallest v key whose x reaches that sample's x; every thread counts
-  // its elements at or above it.  Too few candidates (fewer than k, the
-  // slice not exhausted): r doubles and the registers are counted again. ----
-  const int n_s = (c1 - c0 + kSampleStride - 1) / kSampleStride;
-  const long long kk = (k_req + kSampleStride - 1) / kSampleStride;
-  int r = static_cast<int>(min<long long>(n_s, kk + 3));
-  uint32_t n = 0, mine = 0, incl = 0, bound = 0;
-  while (true) {
-    if (wave == 0) {
-      uint32_t key[kSampleRegs];  // sample keys; 0 (a NaN's key) past the samples
+  // ---- bound: a key that at least k of the threads' maxima reach, then the
+  // smallest key with that key's x ----
+  const uint32_t kk = static_cast<uint32_t>(k_req);
+  const uint32_t enough = kk + (kk >> 3) + 4u;  // a few more than k will do
+  // The smallest key with x >= lo's x: the 64 keys down from lo, then, if all
+  // of them have it (a large temperature), 64 keys tested a round.
+  auto widen = [&](uint32_t lo) -> uint32_t {
+    const float xb = unkey(lo) / P.temp;
+    const uint32_t down = lo - min(lo - 1u, static_cast<uint32_t>(lane));
+    const unsigned long long same = __ballot(unkey(down) / P.temp >= xb);
+    if (same != ~0ull)  // (no lane with a NaN bound: keep lo)
+      return lo - min(lo - 1u, static_cast<uint32_t>(max(static_cast<int>(__builtin_ctzll(~same)) - 1, 0)));
+    uint32_t l2 = 0, h2 = lo - min(lo - 1u, 63u);
+    while (h2 - l2 > 1) {
+      const uint32_t step = (h2 - l2 + 63) / 64;
+      const uint32_t k = min(h2, l2 + step * static_cast<uint32_t>(lane + 1));
+      const unsigned long long ge = __ballot(unkey(k) / P.temp >= xb);  // lane 63 tests h2
+      if (ge == 0) break;
+      const int first = static_cast<int>(__builtin_ctzll(ge));
+      h2 = min(h2, l2 + step * static_cast<uint32_t>(first + 1));
+      l2 = first == 0 ? l2 : l2 + step * static_cast<uint32_t>(first);
+    }
+    return max(h2, 1u);
+  };
+  if (wave == 0) {
+    constexpr int kPer = kSliceThreads / 64;
+    uint32_t t[kPer], top = 0;
 #pragma unroll
-      for (int q = 0; q < kSampleRegs; ++q) {
-        const int j = q * 64 + lane;
-        key[q] = j < n_s ? sh.samp[j] : 0u;
-      }
-      uint32_t best = 0;
-      for (int it = 0; it < min(r, n_s); ++it) {  // remove the largest r - 1 times, one copy each
-        uint32_t m = 0;
+    for (int q = 0; q < kPer; ++q) {
+      t[q] = sh.tmax[q * 64 + lane];
+      top = max(top, t[q]);
+    }
+    top = wave_max_u32(top);
+    auto reach = [&](uint32_t k) {  // maxima at or above k (uniform)
+      uint32_t c = 0;
 #pragma unroll
-        for (int q = 0; q < kSampleRegs; ++q) m = key[q] > m ? key[q] : m;
-        best = wave_max_u32(m);
-        const unsigned long long holders = __ballot(m == best);
-        if (lane == static_cast<int>(__builtin_ctzll(holders))) {
-          bool done = false;
-#pragma unroll
-          for (int q = 0; q < kSampleRegs; ++q)
-            if (!done && key[q] == best) {
-              key[q] = 0u;
-              done = true;
-            }
+      for (int q = 0; q < kPer; ++q) c += static_cast<uint32_t>(__popcll(__ballot(t[q] >= k)));
+      return c;
+    };
+    uint32_t bound = 0u;  // fewer than k threads with elements: see below
+    if (reach(1u) >= kk) {
+      // reach(lo) >= k > reach(hi), unless hi is the largest key there is.
+      uint32_t lo = 1u, hi = top == 0xffffffffu ? top : top + 1u;
+      if (reach(hi) >= kk) lo = hi;
+      // Most rows' maxima lie within a few binades of the largest.
+      else if (top > (3u << 23) && reach(top - (3u << 23)) >= kk) lo = top - (3u << 23);
+      while (hi - lo > 1u) {
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        const uint32_t c = reach(mid);
+        if (c >= kk) {
+          lo = mid;
+          if (c <= enough) break;
+        } else {
+          hi = mid;
         }
       }
-      // The smallest key k in (0, best] with unkey(k) / temp >= unkey(best) /
-      // temp (key 0 is a NaN's: never): 64 keys tested a round, one a lane.
-      const float xb = unkey(best) / P.temp;
-      uint32_t lo = 0, hi = best;
-      while (hi - lo > 1) {
-        const uint32_t step = (hi - lo + 63) / 64;
-        const uint32_t k = min(hi, lo + step * static_cast<uint32_t>(lane + 1));
-        const unsigned long long t = __ballot(unkey(k) / P.temp >= xb);  // lane 63 tests hi
-        if (t == 0) break;  // only with a NaN bound: keep hi
-        const int first = static_cast<int>(__builtin_ctzll(t));
-        hi = min(hi, lo + step * static_cast<uint32_t>(first + 1));
-        lo = first == 0 ? lo : lo + step * static_cast<uint32_t>(first);
+      bound = widen(lo);
+    }
+    if (lane == 0) sh.bound = bound;
+  }
+  __syncthreads();
+  uint32_t bound = sh.bound;
+  if (bound == 0u) {
+    // A short slice (fewer than k threads hold elements): every element (key 0
+    // is a NaN's: none), or, past the candidates' capacity, the same bisection
+    // over the elements themselves.  Uniform over the workgroup.
+    // (an open row's k is too small for that.)
+    uint32_t lo = 1u, hi = MODE == kModeTopK && c1 - c0 > kSliceCand ? 0xffffffffu : 1u;
+    while (hi - lo > 1u) {
+      const uint32_t mid = lo + ((hi - lo) >> 1);
+      uint32_t c = 0;
+#pragma unroll
+      for (int q = 0; q < kSlots; ++q) c += static_cast<uint32_t>(__popcll(__ballot(rg.key[q] >= mid)));
+      if (lane == 0) sh.zw[wave] = c;
+      __syncthreads();
+      c = 0;
+#pragma unroll
+      for (int w = 0; w < kSliceThreads / 64; ++w) c += static_cast<uint32_t>(sh.zw[w]);
+      __syncthreads();
+      if (c >= kk) {
+        lo = mid;
+        if (c <= enough) break;
+      } else {
+        hi = mid;
       }
-      if (lane == 0) sh.bound = r > n_s ? 0u : hi;  // r past the samples: every element
     }
-    __syncthreads();
-    bound = sh.bound;
-    mine = 0;
-#pragma unroll
-    for (int q = 0; q <= SliceRegs<DT>::kVecs * SliceRegs<DT>::W; ++q)
-      mine += rg.valid(q) && rg.key[q] >= bound ? 1u : 0u;
-    incl = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t o = __shfl_up(incl, d);
-      if (lane >= d) incl += o;
-    }
-    if (lane == 63) sh.wcount[wave] = incl;
-    __syncthreads();
-    n = 0;
-#pragma unroll
-    for (int w = 0; w < kSliceThreads / 64; ++w) n += sh.wcount[w];
-    __syncthreads();  // wcount and bound are rewritten by a retry
-    if (static_cast<long long>(n) >= k_req || static_cast<int>(n) == c1 - c0 || r > n_s) break;
-    r = r == n_s ? n_s + 1 : min(n_s, 2 * r);
+    bound = lo > 1u ? widen(lo) : 1u;
   }
-  uint32_t off = incl - mine;
+  // ---- candidates, in any order (each is placed by its rank below) ----
+  unsigned long long reach[2] = {0ull, 0ull};  // slots at or above the bound
+  static_assert(kSlots <= 128, "two words of slots");
 #pragma unroll
-  for (int w = 0; w < kSliceThreads / 64; ++w) off += w < wave ? sh.wcount[w] : 0u;
-  if (mine) {
+  for (int q = 0; q < kSlots; ++q) reach[q >> 6] |= rg.key[q] >= bound ? 1ull << (q & 63) : 0ull;
 #pragma unroll
-    for (int q = 0; q <= SliceRegs<DT>::kVecs * SliceRegs<DT>::W; ++q) {
-      if (!(rg.valid(q) && rg.key[q] >= bound)) continue;
-      if (off < static_cast<uint32_t>(kSliceCand)) sh.cand[off] = order_key(unkey(rg.key[q]) / P.temp, c0 + rg.elem(q));
-      ++off;
+  for (int h = 0; h < (kSlots + 63) / 64; ++h) {
+    for (unsigned long long left = reach[h]; left; left &= left - 1) {
+      const int e = rg.elem(64 * h + __ffsll(left) - 1);
+      float v = elem_to_f32<DT>(logits_row[c0 + e]);  // (cached; the value its key was made of)
+      if (has_hist && ((sh.seen[e >> 5] >> (e & 31)) & 1u)) v = penalise_seen(P, sh, c0 + e, v);
+      const uint32_t o = atomicAdd(&sh.count, 1u);
+      if (o < static_cast<uint32_t>(kSliceCand)) sh.cand[o] = order_key(v / P.temp, c0 + e);
     }
   }
+  __syncthreads();
+  const uint32_t n = sh.count;
   if (n <= static_cast<uint32_t>(kSliceCand) && tid < 16) sh.cand[n + tid] = 0ull;
   __syncthreads();
   const bool ok = n <= static_cast<uint32_t>(kSliceCand) &&
@@ -877,8 +944,8 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
     const float m = m_row / P.temp;
     unsigned long long z = 0;
 #pragma unroll
-    for (int q = 0; q <= SliceRegs<DT>::kVecs * SliceRegs<DT>::W; ++q) {
-      if (!rg.valid(q)) continue;
+    for (int q = 0; q < kSlots; ++q) {
+      if (!rg.key[q]) continue;
       const float x = unkey(rg.key[q]) / P.temp;
       const float e = expf(x - m);
       if (P.min_p <= 0.f || e >= P.min_p) z += mass_of_e(e);
@@ -953,7 +1020,7 @@ __device__ __forceinline__ bool sliced_lists(const SliceWs &ws, int row, int (&n
 // the one the whole-row computation makes.
 __device__ __forceinline__ int64_t sliced_finish(FinishShared &sh, const SliceWs &ws, int row, const Params &P,
                                                  long long k_req, float u, const int (&n)[kSlices], float m,
-                                                 bool open, int V) {
+                                                 bool open, int V, float head_x, int head_i) {
   const int tid = threadIdx.x;
   // Merge: element j of slice s goes to position j + (number of elements of
   // the other slices earlier in the order), found by binary search in each
@@ -961,14 +1028,21 @@ __device__ __forceinline__ int64_t sliced_finish(FinishShared &sh, const SliceWs
   const int64_t base = static_cast<int64_t>(row) * kSlices * kFastMaxK;
   unsigned long long *lists = sh.lists;
   int total = 0;
+  // (the first 64 of each list, entry tid % 64 of list tid / 64, came with the counts)
+  static_assert(kThreads == 64 * kSlices, "one head entry a thread");
 #pragma unroll
   for (int s = 0; s < kSlices; ++s) {
-    for (int j = tid; j < n[s]; j += kThreads)
+    if (s == tid >> 6 && (tid & 63) < n[s]) lists[s * kFastMaxK + (tid & 63)] = order_key(head_x, head_i);
+    for (int j = 64 + tid; j < n[s]; j += kThreads)
       lists[s * kFastMaxK + j] = order_key(ws.x[base + s * kFastMaxK + j], ws.idx[base + s * kFastMaxK + j]);
     total += n[s];
   }
   __syncthreads();
   const int kept_k = open ? total : static_cast<int>(min<long long>(k_req, total));
+  int step0 = 1;  // the largest power of two within the longest list
+#pragma unroll
+  for (int t = 0; t < kSlices; ++t)
+    while (2 * step0 <= n[t]) step0 *= 2;
   for (int e = tid; e < total; e += kThreads) {  // element e of the lists, concatenated
     int s = 0, j = e, before = 0;  // (list, position) of e; n[] indexed by constants only
 #pragma unroll
@@ -980,18 +1054,22 @@ __device__ __forceinline__ int64_t sliced_finish(FinishShared &sh, const SliceWs
       before += n[t];
     }
     const unsigned long long kj = lists[s * kFastMaxK + j];
-    int pos = j;
+    // Elements of each list earlier than kj: the lists' searches side by side,
+    // one LDS round trip a step for all of them (kj's own list gives j).
+    int earlier[kSlices];
 #pragma unroll
-    for (int t = 0; t < kSlices; ++t) {
-      if (t == s) continue;
-      int lo = 0, hi = n[t];  // count of list t's elements earlier than kj
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (lists[t * kFastMaxK + mid] > kj) lo = mid + 1;
-        else hi = mid;
+    for (int t = 0; t < kSlices; ++t) earlier[t] = 0;
+#pragma unroll 1
+    for (int step = step0; step > 0; step >>= 1) {
+#pragma unroll
+      for (int t = 0; t < kSlices; ++t) {
+        const int at = earlier[t] + step;
+        if (at <= n[t] && lists[t * kFastMaxK + at - 1] > kj) earlier[t] = at;
       }
-      pos += lo;
     }
+    int pos = 0;
+#pragma unroll
+    for (int t = 0; t < kSlices; ++t) pos += earlier[t];
     if (pos < kept_k) {
       sh.cx[pos] = unkey(static_cast<uint32_t>(kj >> 32));
       sh.ci[pos] = static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(kj));
@@ -1105,6 +1183,18 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
   Shared &sh = *reinterpret_cast<Shared *>(smem_raw);
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
+  // The heads of the slices' lists, requested with the parameters and the
+  // counts: one memory round trip instead of three (an entry past its list's
+  // count is not used).
+  float head_x = 0.f, lists_max = 0.f;
+  int head_i = 0, n[kSlices];
+  bool lists_ok = false;
+  if (ws.count) {
+    const int64_t at = (static_cast<int64_t>(row) * kSlices + (tid >> 6)) * kFastMaxK + (tid & 63);
+    head_x = ws.x[at];
+    head_i = ws.idx[at];
+    lists_ok = sliced_lists(ws, row, n, &lists_max);
+  }
   Params P;
   P.temp = temperature[row];
   P.top_k = top_k ? top_k[row] : -1;
@@ -1121,13 +1211,11 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
   const bool topk_s = (stages & kStageTopK) && sliced_row(P.temp, k_request(P.top_k, V));
   const bool open_s = (stages & kStageOpen) && open_row(P.temp, k_request(P.top_k, V), P.top_p, P.min_p);
   if (ws.count && (topk_s || open_s)) {
-    int n[kSlices];
-    float mv;
-    if (sliced_lists(ws, row, n, &mv)) {
+    if (lists_ok) {
       static_assert(sizeof(FinishShared) <= sizeof(Shared), "the finish reuses the row kernel's LDS");
       const int64_t tok = sliced_finish(*reinterpret_cast<FinishShared *>(smem_raw), ws, row, P,
-                                        k_request(P.top_k, V), uniforms ? uniforms[row] : 0.f, n, mv / P.temp,
-                                        open_s, V);
+                                        k_request(P.top_k, V), uniforms ? uniforms[row] : 0.f, n, lists_max / P.temp,
+                                        open_s, V, head_x, head_i);
       if (tok >= 0) {
         if (tid == 0) out[row] = tok;
         return;
@@ -1275,6 +1363,22 @@ struct Args {
   int stages;       // kStageTopK | kStageOpen: the sliced stages to run (with a workspace)
 };
 
+// The sliced stages of a call, NQ vectors of a slice a thread.
+template <int DT, int NQ>
+void launch_slices(const Args &a, int rows, int stages, const SliceWs &ws, hipStream_t stream) {
+  const dim3 grid(rows * kSlices);
+#define SPK_SLICES(MODE)                                                                              \
+  sample_slices_kernel<DT, MODE, NQ><<<grid, kSliceThreads, 0, stream>>>(                             \
+      a.logits, a.row_stride, a.V, a.temperature, a.top_k, a.top_p, a.min_p, a.rep, a.presence,       \
+      a.frequency, a.history, a.hist_stride, a.hist_len, a.hist_len_stride, ws)
+  if (stages & kStageOpen) {  // the row maxima, then the lists and masses
+    SPK_SLICES(kModeOpenMax);
+    SPK_SLICES(kModeOpen);
+  }
+  if (stages & kStageTopK) SPK_SLICES(kModeTopK);
+#undef SPK_SLICES
+}
+
 template <int DT, bool VEC>
 int launch(const Args &a, int rows, hipStream_t stream) {
   static bool attr_set = false;  // per instantiation
@@ -1292,18 +1396,14 @@ int launch(const Args &a, int rows, hipStream_t stream) {
     if (a.workspace && a.stages) {
       ws = slice_ws(a.workspace, rows);
       stages = a.stages;
-      if (stages & kStageOpen) {  // the row maxima, then the lists and masses
-        sample_slices_kernel<DT, kModeOpenMax><<<rows * kSlices, kSliceThreads, 0, stream>>>(
-            a.logits, a.row_stride, a.V, a.temperature, a.top_k, a.top_p, a.min_p, a.rep, a.presence, a.frequency,
-            a.history, a.hist_stride, a.hist_len, a.hist_len_stride, ws);
-        sample_slices_kernel<DT, kModeOpen><<<rows * kSlices, kSliceThreads, 0, stream>>>(
-            a.logits, a.row_stride, a.V, a.temperature, a.top_k, a.top_p, a.min_p, a.rep, a.presence, a.frequency,
-            a.history, a.hist_stride, a.hist_len, a.hist_len_stride, ws);
-      }
-      if (stages & kStageTopK)
-        sample_slices_kernel<DT, kModeTopK><<<rows * kSlices, kSliceThreads, 0, stream>>>(
-            a.logits, a.row_stride, a.V, a.temperature, a.top_k, a.top_p, a.min_p, a.rep, a.presence, a.frequency,
-            a.history, a.hist_stride, a.hist_len, a.hist_len_stride, ws);
+      // Registers for the slice length at hand: a quarter, 5/8 or all of the
+      // largest vocabulary's vectors (bf16: up to 65,536, 163,840 and 262,144
+      // entries).
+      constexpr int kAll = kSliceMaxLen / (Elem<DT>::kVec * kSliceThreads);
+      const int need = (slice_len(a.V) / Elem<DT>::kVec + kSliceThreads - 1) / kSliceThreads;
+      if (need <= kAll / 4) launch_slices<DT, kAll / 4>(a, rows, stages, ws, stream);
+      else if (need <= kAll * 5 / 8) launch_slices<DT, kAll * 5 / 8>(a, rows, stages, ws, stream);
+      else launch_slices<DT, kAll>(a, rows, stages, ws, stream);
     }
   }
   sample_kernel<DT, VEC><<<rows, kThreads, shm, stream>>>(

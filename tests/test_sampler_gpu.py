@@ -121,6 +121,40 @@ def test_sampler_sliced_candidates_give_the_same_tokens(gpu, case, dtype):
     assert sliced == plain
 
 
+# Edges of the slices' bound and of their register sizes (bf16: up to 65,536,
+# 163,840 and 262,144 entries; fp32 the same).
+SLICED_EDGE_CASES = [
+    (12000, 3.0, dict(temperature=1.0, top_k=256)),               # fewer threads with elements than k: over 1,024 elements
+    (5000, 3.0, dict(temperature=1.0, top_k=200, top_p=0.99)),    # the same, every element a candidate
+    (4099, 3.0, dict(temperature=0.9, top_k=40, rep=1.2)),        # a last slice of three elements
+    (65536, 3.0, dict(temperature=1.0, top_k=256)),
+    (65537, 3.0, dict(temperature=1.0, top_k=50)),
+    (163840, 3.0, dict(temperature=0.6, top_k=50, top_p=0.9)),
+    (163841, 3.0, dict(temperature=1.0, top_k=7)),
+    (151936, 1e-38, dict(temperature=3.0e4, top_k=30)),           # many keys share an x
+    (151936, 3.0, dict(temperature=1.0e30, top_k=20)),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", range(len(SLICED_EDGE_CASES)))
+def test_sampler_sliced_bound_edges(gpu, case, dtype):
+    """The sliced top-k stage gives the one-workgroup path's tokens, also with
+    masked (-infinity) logits and fewer finite ones than k in a slice."""
+    V, scale, p = SLICED_EDGE_CASES[case]
+    rng = np.random.default_rng(300 + case)
+    rows = 12
+    logits = (rng.standard_normal((rows, V)) * scale).astype(np.float32)
+    logits[3, rng.random(V) < 0.9] = -np.inf
+    logits[4, 100:] = -np.inf
+    logits[5, : V // 2] = 0.0
+    histories = [rng.integers(0, V, size=rng.integers(0, 60)).tolist() for _ in range(rows)]
+    us = rng.random(rows).astype(np.float32).tolist()
+    plain, _ = _run(gpu, logits, [p] * rows, histories, us, dtype)
+    sliced, _ = _run(gpu, logits, [p] * rows, histories, us, dtype, sliced=True)
+    assert sliced == plain
+
+
 # Rows with no top-k cut (the open stage).  "peaked" logits are N(0, 6^2) (a
 # trained model's kind: the top few hundred tokens hold most of the mass, so
 # the slices decide most rows); flat N(0, 2^2) ones leave the cut past the
