@@ -165,6 +165,31 @@ def load(path: str | None = None) -> ctypes.CDLL:
     return lib
 
 
+_UNBOUND = object()
+_native = _UNBOUND
+
+
+def native():
+    """The Python entry module (csrc/native.cpp) bound to the loaded library, or
+    None where it is not built for this torch: the wrappers' own path then
+    makes the same calls through ctypes."""
+    global _native
+    if _native is _UNBOUND:
+        lib = load()
+        try:
+            from . import _native as mod
+        except ImportError:
+            _native = None
+        else:
+            mod.bind(*(ctypes.cast(getattr(lib, name), _vp).value for name in (
+                "spk_decode_attn", "spk_decode_attn_workspace_bytes", "spk_lif_pack_write_sites",
+                "spk_lif_multistep", "spk_prefill_attn", "spk_embed_rmsnorm", "spk_add_rmsnorm",
+                "spk_rmsnorm_mean_t", "spk_lif_gate_mul", "spk_linear_decode", "spk_mlp_gate_lif",
+                "spk_qkv_rope_lif_pack_kv")))
+            _native = mod
+    return _native
+
+
 def check(rc: int, what: str) -> None:
     """Maps a C-ABI status to the exception the reference raises."""
     if rc == SPK_OK:
@@ -194,7 +219,13 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The current stream's handle without building a Stream object (2 us a call less).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(device: torch.device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

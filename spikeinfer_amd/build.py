@@ -1,4 +1,5 @@
-"""Builds libspikeinfer_amd.so (gfx950) in-tree with hipcc.
+"""Builds libspikeinfer_amd.so (gfx950) in-tree with hipcc, and _native.so (the
+Python entry of the launch-bound operators) with g++.
 
 Usage: ``python -m spikeinfer_amd.build`` (or ``build()`` from Python).  The
 library is a plain C-ABI shared object (see include/spikeinfer_amd.h); it is
@@ -35,6 +36,23 @@ def sources() -> list[str]:
 
 
 OBJ_DIR = os.path.join(HERE, "_build")
+NATIVE_PATH = os.path.join(HERE, "_native.so")
+
+
+def native_command(out: str) -> list[str]:
+    """The g++ line of the Python entry (csrc/native.cpp) against the installed torch."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *(f"-I{i}" for i in includes), "-o", out, os.path.join(CSRC, "native.cpp"),
+            "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
 
 
 def _run(cmd: list[str], verbose: bool) -> None:
@@ -42,20 +60,25 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stderr}")
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed ({res.returncode}):\n{res.stderr}")
 
 
 def build(verbose: bool = False) -> str:
     """Compiles every csrc/*.hip to an object (in parallel, one hipcc per
-    file) and links them into the shared library.  Always recompiles."""
+    file) and links them into the shared library, and csrc/native.cpp into
+    the Python entry module beside it.  Always recompiles."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
     objs = [os.path.join(OBJ_DIR, os.path.basename(s)[:-4] + ".o") for s in srcs]
-    jobs = max(1, min(len(srcs), os.cpu_count() or 1, 16))
+    jobs = max(1, min(len(srcs) + 1, os.cpu_count() or 1, 16))
+    native_tmp = NATIVE_PATH + ".tmp"
     with ThreadPoolExecutor(jobs) as ex:
+        native = ex.submit(_run, native_command(native_tmp), verbose)
         list(ex.map(lambda so: _run([hipcc, *HIPCC_FLAGS, "-c", "-o", so[1], so[0]], verbose),
                     zip(srcs, objs)))
+        native.result()
+    os.replace(native_tmp, NATIVE_PATH)
     tmp = LIB_PATH + ".tmp"
     _run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp, *objs], verbose)
     os.replace(tmp, LIB_PATH)

@@ -12,6 +12,9 @@ import torch
 
 from .. import _lib
 
+# Each operator first offers its arguments to the C++ entry (csrc/native.cpp),
+# which takes their usual form and answers None, having done nothing, otherwise.
+
 _VEC_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 
@@ -27,6 +30,9 @@ def add_rmsnorm(h: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tenso
     ``h``/``delta``/``out`` ``[..., hidden]`` contiguous, ``weight [hidden]``.
     Returns ``out`` (allocated like ``h`` when None).
     """
+    native = _lib.native()
+    if native is not None and (done := native.add_rmsnorm(h, delta, weight, eps, out)) is not None:
+        return done
     dev = _lib.require_gpu(h, delta, weight, out)
     if h.dtype not in _VEC_DTYPES:
         raise ValueError(f"add_rmsnorm: unsupported dtype {h.dtype}")
@@ -60,6 +66,11 @@ def embed_rmsnorm(ids: torch.Tensor, embed: torch.Tensor, weight: torch.Tensor, 
     Returns ``(h, x)``, both ``[T, n, hidden]``: ``h[t] = embed[ids]`` and
     ``x[t] = Qwen2RMSNorm(h[t])``.
     """
+    native = _lib.native()
+    if native is not None and h is None and out is None:
+        done = native.embed_rmsnorm(ids, embed, weight, eps, T)
+        if done is not None:
+            return done
     dev = _lib.require_gpu(ids, embed, weight, h, out)
     if ids.dtype != torch.int64 or ids.ndim != 1 or not ids.is_contiguous():
         raise ValueError("embed_rmsnorm: ids must be a contiguous int64 vector")
@@ -89,6 +100,11 @@ def rmsnorm_mean_t(h: torch.Tensor, weight: torch.Tensor, eps: float,
                    out: torch.Tensor | None = None, delta: torch.Tensor | None = None) -> torch.Tensor:
     """``RMSNorm(h + delta).mean(dim=0)`` for ``h [T, rows, hidden]``
     contiguous (``delta`` optional, same shape; h is not modified)."""
+    native = _lib.native()
+    if native is not None and out is None:
+        done = native.rmsnorm_mean_t(h, weight, eps, delta)
+        if done is not None:
+            return done
     dev = _lib.require_gpu(h, weight, out, delta)
     if h.ndim != 3:
         raise ValueError("rmsnorm_mean_t: expected h as [T, rows, hidden]")
@@ -145,6 +161,12 @@ def qkv_rope_lif_pack(
             receives the k and v words too, token by token.
     Returns ``q_packed``.
     """
+    native = _lib.native()
+    if native is not None and dense is None and positions is not None:
+        pk, pv = kv_packed if kv_packed is not None else (None, None)
+        if native.qkv_rope_lif_pack(qkv, cos, sin, beta, threshold, k_cache, v_cache, slot_mapping, num_q_heads,
+                                    num_kv_heads, head_dim, q_packed, n_q, positions, pk, pv):
+            return q_packed
     dev = _lib.require_gpu(qkv, cos, sin, beta, threshold, k_cache, v_cache, slot_mapping, q_packed,
                            positions)
     if qkv.ndim != 3 or qkv.stride(-1) != 1:
@@ -271,6 +293,11 @@ def lif_gate_mul(gate_up: torch.Tensor, beta: torch.Tensor, threshold: torch.Ten
 
     Returns ``[T, rows, I]`` contiguous in gate_up's dtype.
     """
+    native = _lib.native()
+    if native is not None and out is None:
+        done = native.lif_gate_mul(gate_up, beta, threshold)
+        if done is not None:
+            return done
     dev = _lib.require_gpu(gate_up, beta, threshold, out)
     if gate_up.ndim != 3 or gate_up.stride(-1) != 1:
         raise ValueError("gate_up must be [T, rows, 2I] with a contiguous channel axis")
@@ -333,6 +360,9 @@ def linear_decode(x: torch.Tensor, w_packed: torch.Tensor, bias: torch.Tensor | 
     from :func:`pack_linear`'s weight, into ``out`` when given (contiguous);
     None when the shape is outside the kernel's range (the caller then uses
     ``F.linear``)."""
+    native = _lib.native()
+    if native is not None and (done := native.linear_decode(x, w_packed, bias, out)) is not None:
+        return done
     dev = _lib.require_gpu(x, w_packed, bias, out)
     if x.dtype != torch.bfloat16 or w_packed.ndim != 2 or w_packed.shape[1] != x.shape[-1]:
         raise ValueError("x must be bf16 [..., K] and w_packed [N, K]")
@@ -364,6 +394,11 @@ def mlp_gate_lif(x: torch.Tensor, w_packed: torch.Tensor, beta: torch.Tensor,
     Returns ``[T, n_tok, I]``, or None when the shape is outside the kernel's
     range (the caller then runs the GEMM and :func:`lif_gate_mul`).
     """
+    native = _lib.native()
+    if native is not None and out is None:
+        done = native.mlp_gate_lif(x, w_packed, beta, threshold)
+        if done is not None:
+            return done
     dev = _lib.require_gpu(x, w_packed, beta, threshold, out)
     if x.ndim != 3 or x.dtype != torch.bfloat16:
         raise ValueError("x must be a bf16 [T, n_tok, hidden] tensor")

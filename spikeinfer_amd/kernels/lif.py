@@ -36,6 +36,11 @@ def lif_multistep(x, beta, threshold, mem0=None, out_dtype=None, return_membrane
     Threshold > 0 is a precondition checked once by :func:`validate_thresholds`
     (a per-call check would need a device sync, illegal under graph capture).
     """
+    if mem0 is None and (out_dtype is None or out_dtype == x.dtype):
+        native = _lib.native()
+        done = native.lif(x, beta, threshold, bool(return_membrane)) if native is not None else None
+        if done is not None:
+            return done
     assert x.ndim >= 2, "expected [T, *mid, N]"
     N = x.shape[-1]
     assert beta.numel() == N and threshold.numel() == N, (
@@ -177,6 +182,9 @@ def lif_pack_write_sites(sites, slot_mapping: torch.Tensor | None = None) -> Non
     sites of attention.py:138-149 / modeling_fast.py:132-134.
     """
     sites = list(sites)
+    native = _lib.native()
+    if native is not None and native.lif_sites(sites, slot_mapping):
+        return
     if not 1 <= len(sites) <= 4:
         raise ValueError(f"lif_pack_write_sites takes 1 to 4 sites, got {len(sites)}")
     if slot_mapping is not None:

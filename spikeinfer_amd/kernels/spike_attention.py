@@ -66,6 +66,12 @@ def paged_spike_attn_decode(
     scratch (``uint8``, at least :func:`decode_attn_workspace_bytes`); by
     default it comes from torch's caching allocator, which is capture-safe.
     """
+    native = _lib.native()
+    if native is not None:  # the usual form of the arguments, checked and launched in C++
+        done = native.decode_attn(q_packed, k_cache, v_cache, block_tables, seq_lens, head_dim, block_size,
+                                  num_q_heads, num_kv_heads, out, dtype, workspace)
+        if done is not None:
+            return done
     T, n_seqs, n_heads, words = q_packed.shape
     if words != packed_width(head_dim):
         raise ValueError(f"q has {words} words, expected {packed_width(head_dim)}")
@@ -240,6 +246,9 @@ def paged_spike_attn_prefill(
     with ``table`` None (``ctx`` 0), in slot ``q_row + j`` of ``k_words``.
     ``out_row - q_row`` is the same for all chunks.
     """
+    native = _lib.native()
+    if native is not None and native.prefill(q_packed, k_words, v_words, chunks, out, head_dim, block_size):
+        return out
     T, _, n_heads, words = q_packed.shape
     dev = _lib.require_gpu(q_packed, k_words, v_words, out)
     for name, t in (("q_packed", q_packed), ("k", k_words), ("v", v_words)):
