@@ -30,6 +30,15 @@
 //     order through LDS (deterministic).
 // Grid: token groups x 64 column ranges; the token groups of one range are
 // consecutive on one XCD (block b -> XCD b % 8), so W comes from HBM once.
+// With one or two token groups 64 ranges leave half of the CUs or more idle:
+// there the pairs go over 256 or 128 ranges (SPREAD), a wave taking one chain of
+// the 64-range split, so the sums are bit for bit the same at every batch size
+// (one decoder layer in a hipGraph with its own weights, hidden 896, inter 4864,
+// T = 4: 1 to 16 tokens 12.9 -> 10.2 us, 32 tokens 13.2 -> 11.8; 48 tokens at 80
+// ranges 13.2 -> 13.4, so from three groups on the 64 ranges stay.  What is left
+// at 5 tokens is latency: the launch, x into LDS, a chain of up to three
+// quarters, the sums.  Eighths of K per wave with x in registers took 8.1 there,
+// but 16.9 against 13.9 at 64 tokens, and all batches must add alike).
 #include "common.hpp"
 #include "lif_math.hpp"
 #include "norm_rows.hpp"
@@ -59,15 +68,25 @@ static_assert(kStageOff + kWaves * kStageBytes <= kLdsBytes, "slots and staging 
 // KB: lane l's 16 bytes are W[row][32ks + 8(l/16) .. +7], row = 16p + l%16
 // (+ I for up).
 
+// Does a chain of products start at K-quarter q of pair p?  (With kRanges ranges
+// the eight waves of a workgroup take equal shares of its units in order; each
+// pair's part of a share is one chain.)
+__device__ inline bool starts_chain(int p, int q, int P) {
+  const int r = ((p + 1) * kRanges - 1) / P, first = r * P / kRanges;
+  const int U = 4 * ((r + 1) * P / kRanges - first), v = 4 * (p - first) + q;
+  return q == 0 || (kWaves * v + U - 1) / U * U / kWaves == v;
+}
+
+// SPREAD: R > kRanges column ranges, one chain per wave.
 // T is a template parameter: a runtime test per row tile would put branches
 // between the MFMAs (and the accumulator copies they bring cost registers).
 // NORM: the x rows are add_rmsnorm(nin.h, nin.delta, nin.w), computed in the
 // prologue; the workgroups of the last column range (never empty) write h +
 // delta to nin.h_out.
-template <int KQ, int T, bool NORM>
+template <int KQ, int T, bool NORM, bool SPREAD>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void mlp_gate_lif_kernel(
     const uint16_t *x, const v4u *wp, const float *beta_p, const float *th_p, uint16_t *y, int n,
-    int I, int MG, NormIn nin) {
+    int I, int MG, int R, NormIn nin) {
   constexpr int KS = 4 * KQ;       // k-steps of 32 (H = 32 KS)
   constexpr int H = 32 * KS;
   constexpr int kChunks = 4 * KS;  // 16-byte chunks per x row
@@ -76,7 +95,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   const int b = blockIdx.x, xcd = b & 7, s = b >> 3;
   const int m = s % MG, r = (s / MG) * 8 + xcd;
   const int P = I / 16;
-  const int p0 = r * P / kRanges, np = (r + 1) * P / kRanges - p0;
+  const int p0 = r * P / R, np = (r + 1) * P / R - p0;
   if (np <= 0) return;  // uniform over the workgroup
   // The LIF parameters of the pair this wave finishes (wave e < np: pair
   // p0 + e), loaded first so their latency hides under the whole K loop.
@@ -84,10 +103,28 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   const float beta = clamp01(beta_p[ch]);
   const float th = th_p[ch];
 
-  // Units (pair, K-quarter): wave w takes [u0, u1), at most 4 of them, over at
-  // most two pairs.
+  // Units (pair, K-quarter): wave w takes [bound[w], bound[w + 1]), at most 4 of
+  // them, over at most two pairs.
   const int U = 4 * np;
-  const int u0 = wave * U / kWaves, u1 = (wave + 1) * U / kWaves, nu = u1 - u0;
+  uint64_t starts = 0;  // SPREAD: bit u, a chain starts at unit u (lane u looks)
+  if constexpr (SPREAD) starts = __ballot(lane < U && starts_chain(p0 + (lane >> 2), lane & 3, P));
+  auto next_start = [&] {
+    const int u = starts ? __builtin_ctzll(starts) : U;
+    starts &= starts - 1;
+    return u;
+  };
+  int u0 = 0, u1 = 0;
+  if constexpr (SPREAD) {
+    const uint64_t all = starts;
+    for (int w = 0; w < wave; ++w) starts &= starts - 1;
+    u0 = next_start();
+    u1 = next_start();
+    starts = all;
+  } else {
+    u0 = wave * U / kWaves;
+    u1 = (wave + 1) * U / kWaves;
+  }
+  const int nu = u1 - u0;
   // W arrives with nontemporal loads (graph of 24 distinct weights: 15.66
   // -> 15.10 us a launch).
   auto load_unit = [&](int u, v4u (&dst)[KQ][2]) {
@@ -102,7 +139,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   const int rows = T * kTok;
   if constexpr (NORM) {
     norm_rows<kWaves, T * kTok / kWaves>(
-        nin, rows, H, r == kRanges - 1, wave, lane,
+        nin, rows, H, r == R - 1, wave, lane,
         [&](int rr) { return static_cast<int64_t>(rr >> 4) * n + min(m * kTok + (rr & 15), n - 1); },
         [&](int rr) { return m * kTok + (rr & 15) < n; },
         [&](int rr, int v, const NormRowBf16::v8u16 &yv) {
@@ -155,7 +192,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     }
   };
   auto next_pair = [&](int u) {  // unit u starts a new pair after the wave's first
-    if (u > u0 && (u % 4) == 0) {
+    if (!SPREAD && u > u0 && (u % 4) == 0) {  // (a chain stays within a pair)
 #pragma unroll
       for (int t = 0; t < kMaxT; ++t) {
         saveg[t] = accg[t];
@@ -213,8 +250,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   for (int t = 0; t < kMaxT; ++t)
 #pragma unroll
     for (int j = 0; j < 4; ++j) sg[t][j] = su[t][j] = 0.f;
+  int next = SPREAD ? next_start() : 0;
   for (int w = 0; w < kWaves; ++w) {
-    const int a0 = w * U / kWaves, a1 = (w + 1) * U / kWaves;
+    const int a0 = SPREAD ? next : w * U / kWaves, a1 = SPREAD ? next_start() : (w + 1) * U / kWaves;
+    next = a1;
     if (a1 <= a0) continue;
     const int pf = a0 / 4, pl = (a1 - 1) / 4;
     int slot = -1;
@@ -277,6 +316,11 @@ __global__ __launch_bounds__(256) void mlp_gate_pack_kernel(const uint16_t *w, v
   }
 }
 
+// Column ranges of a launch: one workgroup per CU for one or two token groups.
+// A range then holds at most 8 chains (128 ranges) or 5 (256), a wave each, for
+// every number of pairs that mlp_shape_ok lets through (counted for all of them).
+inline int ranges_for(int MG) { return MG > 2 ? kRanges : 256 / MG; }
+
 }  // namespace mlp
 
 static bool mlp_shape_ok(int T, int n_tok, int hidden, int inter) {
@@ -323,27 +367,30 @@ static int mlp_gate_launch(const void *x, const NormIn *nin, const void *w_packe
   if (reinterpret_cast<uintptr_t>(y) & 15)  // (the tile rows go out as 16-byte stores)
     return fail(SPK_EUNSUPPORTED, "mlp_gate_lif: y must be 16-byte aligned");
   const int MG = (n_tok + mlp::kTok - 1) / mlp::kTok;
-  const dim3 grid(MG * mlp::kRanges);
+  const int R = nin ? mlp::kRanges : mlp::ranges_for(MG);
+  const dim3 grid(MG * R);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto *xp = static_cast<const uint16_t *>(x);
   const auto *wp = static_cast<const mlp::v4u *>(w_packed);
   auto *yp = static_cast<uint16_t *>(y);
   const NormIn none{};
-#define SPK_MLP_LAUNCH1(KQ, TT, NORM)                                                                \
+#define SPK_MLP_LAUNCH1(KQ, TT, NORM, SPREAD)                                                                \
   {                                                                                                \
     static bool attr = false;                                                                      \
     if (!attr) {                                                                                   \
-      if (hipFuncSetAttribute(reinterpret_cast<const void *>(mlp::mlp_gate_lif_kernel<KQ, TT, NORM>), \
+      if (hipFuncSetAttribute(reinterpret_cast<const void *>(mlp::mlp_gate_lif_kernel<KQ, TT, NORM, SPREAD>), \
                               hipFuncAttributeMaxDynamicSharedMemorySize, mlp::kLdsBytes) != hipSuccess) \
         return fail(SPK_EHIP, "mlp_gate_lif: cannot reserve %d bytes of LDS", mlp::kLdsBytes);  \
       attr = true;                                                                                 \
     }                                                                                              \
-    mlp::mlp_gate_lif_kernel<KQ, TT, NORM><<<grid, mlp::kThreads, mlp::kLdsBytes, s>>>(             \
+    mlp::mlp_gate_lif_kernel<KQ, TT, NORM, SPREAD><<<grid, mlp::kThreads, mlp::kLdsBytes, s>>>(             \
         xp, wp, static_cast<const float *>(beta), static_cast<const float *>(threshold), yp, n_tok,  \
-        inter, MG, nin ? *nin : none);                                                             \
+        inter, MG, R, nin ? *nin : none);                                                            \
   }
 #define SPK_MLP_LAUNCH(KQ, TT)                                                                       \
-  if (nin) SPK_MLP_LAUNCH1(KQ, TT, true) else SPK_MLP_LAUNCH1(KQ, TT, false)
+  if (nin) SPK_MLP_LAUNCH1(KQ, TT, true, false)                                                       \
+  else if (R > mlp::kRanges) SPK_MLP_LAUNCH1(KQ, TT, false, true)                                     \
+  else SPK_MLP_LAUNCH1(KQ, TT, false, false)
 #define SPK_MLP_CASE(KQ)                                                                             \
   case KQ:                                                                                         \
     if (T == 1) SPK_MLP_LAUNCH(KQ, 1)                                                             \

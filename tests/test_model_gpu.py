@@ -299,6 +299,25 @@ def test_mlp_gate_lif_matches_reference(gpu, T, n, H, I):
     assert bool((d <= tol).all()), f"max product difference {float(d.max())}"
 
 
+@pytest.mark.parametrize("T,H,I", [(4, 896, 4864), (4, 512, 1024), (4, 1024, 8192), (2, 640, 1056), (1, 768, 3008),
+                                   (3, 896, 6160)])
+def test_mlp_gate_lif_small_batch_is_bit_identical(gpu, T, H, I):
+    """One and two token groups spread over more column ranges; every row keeps
+    the bits that it has in a batch of 64 (at 64 ranges): the fewest and the most
+    pairs, one to five and eight a range, edges of the token groups."""
+    from spikeinfer_amd.kernels.decoder_ops import mlp_gate_lif, pack_gate_up
+
+    g = torch.Generator(device=gpu).manual_seed(T + H + I)
+    x = (torch.randn((T, 64, H), generator=g, device=gpu) * 1.2).bfloat16()
+    wp = pack_gate_up((torch.randn((2 * I, H), generator=g, device=gpu) * 0.05).bfloat16())
+    beta = 0.6 + 0.4 * torch.rand(I, generator=g, device=gpu)
+    th = 0.5 + torch.rand(I, generator=g, device=gpu)
+    want = mlp_gate_lif(x, wp, beta, th)
+    for n in (1, 15, 16, 17, 32, 33):
+        print(f"mlp_gate_lif small batch T={T} H={H} I={I} n={n}", flush=True)
+        assert torch.equal(mlp_gate_lif(x[:, :n].contiguous(), wp, beta, th), want[:, :n])
+
+
 def test_mlp_gate_lif_unsupported_shapes_return_none(gpu):
     from spikeinfer_amd.kernels.decoder_ops import mlp_gate_lif, pack_gate_up
 
