@@ -462,10 +462,14 @@ static int launch_linear_tiled(const void *x, const void *w_packed, const void *
   // otherwise.  Measured (graph of 24 distinct weights, K = 896): M = 32:
   // q/k/v 5.46 -> 4.25 us, o 5.17 -> 4.11 us; M = 256: o (N = 896) 5.37 ->
   // 5.14 us, q/k/v (N = 1152, three tiles a range) 6.90 -> 6.45 us.  The sum
-  // of every element (eight K parts in order) is the same either way.
+  // of every element (eight K parts in order) is the same either way.  The
+  // count is rounded down to a multiple of 8: rounded up, 3, 5, 6 or 7 row
+  // groups made 264 to 288 workgroups, the last ones a second pass over the
+  // chip (q/k/v at 96 rows 5.5 -> 4.2 us, at 192 rows 5.6 -> 5.1; N = 1536,
+  // K = 1024 at 160 rows 10.3 -> 5.4).
   const int P = N / 16;
   auto ranges = [&](int MG, int mu) {
-    int R = ((256 / MG) + 7) / 8 * 8;
+    int R = 256 / MG / 8 * 8;
     if (R < 8) R = 8;
     while (R * mu < P) R += 8;
     return R;
@@ -511,11 +515,14 @@ extern "C" int spk_linear_decode(const void *x, const void *w_packed, const void
   if (K > lin::kParts * lin::kMaxPartSteps * 32 && !bias && M >= 1 && M <= 4 * lin::kRows &&
       N >= 16 && N % 16 == 0 && K % 128 == 0 &&
       static_cast<int64_t>(lin::kTallRows) * K * 2 <= lin::kLdsBytes) {
-    // Long K: 16-row groups, 3-4 tiles per range.
+    // Long K: 16-row groups, at most 4 tiles per range.  About 256 workgroups,
+    // rounded down to ranges in multiples of 8: one workgroup fills a CU's LDS, and
+    // the 264 to 288 of a rounded-up count took a second pass (N = 896, K = 4864:
+    // 80 rows 12.1 -> 9.0 us, 96 rows 13.8 -> 9.0, 160 rows 15.9 -> 11.0).
     if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(w_packed) & 15))
       return fail(SPK_EINVAL, "linear_decode: x and packed weights must be 16-byte aligned");
     const int MG = (M + lin::kTallRows - 1) / lin::kTallRows;
-    int R = ((256 / MG) + 7) / 8 * 8;
+    int R = 256 / MG / 8 * 8;
     while (R * 4 < N / 16) R += 8;
     static bool attr = false;
     if (!attr) {

@@ -328,6 +328,23 @@ def test_mlp_gate_lif_unsupported_shapes_return_none(gpu):
         assert mlp_gate_lif(x, pack_gate_up(w), b, b) is None
 
 
+@pytest.mark.parametrize("N,K,bias", [(896, 4864, False), (1152, 896, True), (1536, 1024, True), (16, 2048, False),
+                                      (4112, 1408, False), (16, 128, False)])
+def test_linear_decode_rows_do_not_depend_on_the_batch(gpu, N, K, bias):
+    """Every row keeps the bits that it has in a batch of at most 64 rows, at the
+    row counts where the number of row groups does not divide 256 workgroups."""
+    from spikeinfer_amd.kernels.decoder_ops import linear_decode, pack_linear
+
+    g = torch.Generator(device=gpu).manual_seed(N + K)
+    x = torch.randn((1, 256, K), generator=g, device=gpu).bfloat16()
+    wp = pack_linear((torch.randn((N, K), generator=g, device=gpu) * 0.05).bfloat16())
+    b = (torch.randn(N, generator=g, device=gpu) * 0.1).bfloat16() if bias else None
+    want = torch.cat([linear_decode(x[:, i:i + 64].contiguous(), wp, b) for i in range(0, 256, 64)], 1)
+    for M in (65, 80, 96, 113, 127, 129, 160, 161, 192, 224, 256):
+        print(f"linear_decode rows M={M} N={N} K={K}", flush=True)
+        assert torch.equal(linear_decode(x[:, :M].contiguous(), wp, b), want[:, :M])
+
+
 @pytest.mark.parametrize("M,N,K,bias", [(256, 1152, 896, True), (256, 896, 896, False),
                                          (44, 1152, 896, True), (4, 896, 896, False),
                                          (130, 512, 1280, True), (64, 48, 128, False),
