@@ -27,6 +27,7 @@
 #include "common.hpp"
 #include "lif_math.hpp"
 #include "norm_rows.hpp"
+#include "stage_rows.hpp"
 
 namespace spk {
 namespace lin {
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(RT == 
     }
   }
 
-  // x rows m0..m0+16RT-1 (clamped to M - 1) into LDS, chunk c of row rr at c ^ (rr % 16).
+  // x rows m0..m0+16RT-1 into LDS, chunk c of row rr at c ^ (rr % 16).
   if constexpr (NORM) {
     norm_rows<kWaves, kRows / kWaves>(
         nin, kRows, K, r == R - 1, wave, lane, [&](int rr) { return static_cast<int64_t>(min(m0 + rr, M - 1)); },
@@ -112,15 +113,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(RT == 
           *reinterpret_cast<NormRowBf16::v8u16 *>(smem + rr * (kChunks * 16) + 16 * (v ^ (rr & 15))) = yv;
         });
   } else {
-    const int total = kR * kChunks;  // a multiple of 64 (K % 128 == 0)
-    for (int base = wave * 64; base < total; base += kWaves * 64) {
-      const int g = base + lane;
-      const int rr = g / kChunks, pc = g - rr * kChunks;
-      const int c = pc ^ (rr & 15);
-      const int row = min(m0 + rr, M - 1);
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const void *>(x + static_cast<int64_t>(row) * K + 8 * c),
-                                       (SPK_LDS void *)(smem + base * 16), 16, 0, 0);
-    }
+    stage_rows<kWaves>(smem, x, min(kR, M - m0), kChunks, wave, lane, [](int) { return true; },
+                       [&](int rr) { return static_cast<int64_t>(m0 + rr); });
   }
   __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0)
   __syncthreads();
@@ -330,11 +324,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 }
 
 // Long K (the down projection, K = 4864) at M <= 256: 16 rows of x per
-// workgroup (16 * K * 2 <= 160 KB of LDS), 3-4 column tiles per workgroup, and
-// the 8 waves split K into eighths.  Each wave streams its k-steps of W in
-// chunks of 4 through a double buffer (branch-free: a chunk past the wave's
-// range multiplies a zero B), then the eight partials of each tile are added
-// in wave order through LDS.
+// workgroup (16 * K * 2 <= 160 KB of LDS), at most 4 column tiles per
+// workgroup, and the 8 waves split K into eighths.  Bound by moving x and W into
+// the CU (467 KB at 128 rows).  Each wave streams its k-steps of W in chunks of 4
+// through two buffers and requests the first two right behind its share of x,
+// before it waits for x; then the eight partials of each tile are added in wave
+// order through LDS.
+// Measured (graph of 24 distinct weights, N = 896), against W requested after
+// x, chunks past the wave's range multiplied by zero, and a division per load of
+// x (stage_rows): 4 rows 7.2 -> 5.3 us, 20 rows 7.1 -> 5.6, 64 rows 7.1 -> 6.4,
+// 128 rows 9.2 -> 7.6, 256 rows 16.9 -> 11.4.  All of a wave's W in registers at
+// once was slower with one tile (4 rows 6.1) and no faster with two.
 constexpr int kTallRows = 16;
 constexpr int kTallChunk = 4;  // k-steps per chunk
 template <int NP>
@@ -344,7 +344,8 @@ __device__ __forceinline__ void linear_tall_run(const v4u *wp, uint16_t *y, int 
   const int kChunks = 4 * KS;  // 16-byte chunks per x row
   const int r16 = lane & 15, kq = lane >> 4;
   const int k0 = wave * KS / kWaves, nk = (wave + 1) * KS / kWaves - k0;
-  const int nc = ((nk + kTallChunk - 1) / kTallChunk + 1) & ~1;  // chunks, even
+  const int nc = (nk + kTallChunk - 1) / kTallChunk;
+  // (a k-step past the wave's last re-reads it and is not multiplied)
   auto load = [&](int c, v4u (&b)[kTallChunk][NP]) {
 #pragma unroll
     for (int j = 0; j < kTallChunk; ++j) {
@@ -360,23 +361,28 @@ __device__ __forceinline__ void linear_tall_run(const v4u *wp, uint16_t *y, int 
 #pragma unroll
     for (int j = 0; j < kTallChunk; ++j) {
       const int kk = c * kTallChunk + j;
-      const int ks = k0 + min(kk, nk - 1);
-      const int ch = 4 * ks + kq;
+      if (kk >= nk) break;  // (uniform over the wave)
+      const int ch = 4 * (k0 + kk) + kq;
       const v8b a = *reinterpret_cast<const v8b *>(smem + r16 * (kChunks * 16) + 16 * (ch ^ r16));
 #pragma unroll
-      for (int t = 0; t < NP; ++t) {
-        const v4u bz = kk < nk ? b[j][t] : v4u{0u, 0u, 0u, 0u};
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(v8b, bz), acc[t], 0, 0, 0);
-      }
+      for (int t = 0; t < NP; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(v8b, b[j][t]), acc[t], 0, 0, 0);
     }
   };
   v4u bA[kTallChunk][NP], bB[kTallChunk][NP];
   load(0, bA);
+  load(1, bB);
+  // vmcnt counts in issue order: at most the W loads outstanding means that
+  // every x chunk of this wave has landed.
+  constexpr int kFirst = 2 * kTallChunk * NP;
+  static_assert(kFirst <= 63, "vmcnt holds 6 bits");
+  __builtin_amdgcn_s_waitcnt(0x3f70 | (kFirst & 15) | ((kFirst >> 4) << 14));
+  __syncthreads();
   for (int c = 0; c < nc; c += 2) {
-    load(c + 1, bB);
     compute(c, bA);
-    load(c + 2, bA);  // past the end: clamped re-reads, never used
+    if (c + 2 < nc) load(c + 2, bA);
     compute(c + 1, bB);
+    if (c + 3 < nc) load(c + 3, bB);
   }
   __syncthreads();  // every wave is done with the x rows: the LDS takes the partials
   float *slots = reinterpret_cast<float *>(smem);
@@ -409,16 +415,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   const int p0 = r * P / R, np = (r + 1) * P / R - p0;
   if (np <= 0) return;  // uniform over the workgroup
   const int m0 = m * kTallRows;
-  for (int base = wave * 64; base < kTallRows * kChunks; base += kWaves * 64) {
-    const int g = base + lane;
-    const int rr = g / kChunks, pc = g - rr * kChunks;
-    const int c = pc ^ (rr & 15);
-    const int row = min(m0 + rr, M - 1);
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const void *>(x + static_cast<int64_t>(row) * K + 8 * c),
-                                     (SPK_LDS void *)(smem + base * 16), 16, 0, 0);
-  }
-  __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0)
-  __syncthreads();
+  stage_rows<kWaves>(smem, x, min(kTallRows, M - m0), kChunks, wave, lane, [](int) { return true; },
+                     [&](int rr) { return static_cast<int64_t>(m0 + rr); });
   if (np == 4) linear_tall_run<4>(wp, y, M, N, KS, m0, p0, smem);
   else if (np == 3) linear_tall_run<3>(wp, y, M, N, KS, m0, p0, smem);
   else if (np == 2) linear_tall_run<2>(wp, y, M, N, KS, m0, p0, smem);

@@ -34,7 +34,7 @@
 // there the pairs go over 256 or 128 ranges (SPREAD), a wave taking one chain of
 // the 64-range split, so the sums are bit for bit the same at every batch size
 // (one decoder layer in a hipGraph with its own weights, hidden 896, inter 4864,
-// T = 4: 1 to 16 tokens 12.9 -> 10.2 us, 32 tokens 13.2 -> 11.8; 48 tokens at 80
+// T = 4: 5 tokens 12.9 -> 10.2 us, 32 tokens 13.2 -> 11.8; 48 tokens at 80
 // ranges 13.2 -> 13.4, so from three groups on the 64 ranges stay.  What is left
 // at 5 tokens is latency: the launch, x into LDS, a chain of up to three
 // quarters, the sums.  Eighths of K per wave with x in registers took 8.1 there,
@@ -42,6 +42,7 @@
 #include "common.hpp"
 #include "lif_math.hpp"
 #include "norm_rows.hpp"
+#include "stage_rows.hpp"
 
 namespace spk {
 namespace mlp {
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
       for (int g = 0; g < 2; ++g) dst[ks][g] = __builtin_nontemporal_load(src + (ks * 2 + g) * 64);
   };
   // x rows of the token group into LDS: row rr = 16 t + i holds token 16m + i
-  // (clamped to n - 1) at timestep t; chunk c of it at chunk c ^ (rr % 16).
+  // (none past n - 1) at timestep t; chunk c of it at chunk c ^ (rr % 16).
   const int rows = T * kTok;
   if constexpr (NORM) {
     norm_rows<kWaves, T * kTok / kWaves>(
@@ -146,16 +147,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
           *reinterpret_cast<NormRowBf16::v8u16 *>(smem + rr * (kChunks * 16) + 16 * (v ^ (rr & 15))) = yv;
         });
   } else {
-    const int total = rows * kChunks;  // a multiple of 64
-    for (int base = wave * 64; base < total; base += kWaves * 64) {
-      const int g = base + lane;
-      const int rr = g / kChunks, pc = g - rr * kChunks;
-      const int c = pc ^ (rr & 15);
-      const int t = rr >> 4, tok = min(m * kTok + (rr & 15), n - 1);
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const void *>(x + (static_cast<int64_t>(t) * n + tok) * H + 8 * c),
-          (SPK_LDS void *)(smem + base * 16), 16, 0, 0);
-    }
+    stage_rows<kWaves>(
+        smem, x, rows, kChunks, wave, lane, [&](int rr) { return m * kTok + (rr & 15) < n; },
+        [&](int rr) { return static_cast<int64_t>(rr >> 4) * n + m * kTok + (rr & 15); });
   }
   // Then the first two units of W; the wait below lets those stay in flight
   // (vmcnt counts in issue order, so at most their loads outstanding means

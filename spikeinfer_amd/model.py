@@ -119,10 +119,14 @@ class SpikingDecoder:
         self.fused_mlp_max_tokens = 64
         # The same batches run the q/k/v and o projections through
         # linear_decode (repacked copies of w_qkv, w_o); False keeps F.linear.
-        # The down projection (long K) goes there only up to small_down_max_rows
-        # rows (T * tokens): beyond, the library GEMM is faster.
+        # The down projection (long K) goes there up to small_down_max_rows rows
+        # (T * tokens).  With hidden <= 1024 all 256 rows are one pass over the
+        # chip (hidden 896, inter 4864: 128 rows 7.6 us against the library
+        # GEMM's 9.9, 160 rows 9.0 against 11.0, 192 and 256 rows equal at 10.9
+        # and 11.4); wider, the library GEMM is faster past 128 rows (256 rows,
+        # 1536 x 5120: 19.9 us against 27.1).
         self.small_linear = True
-        self.small_down_max_rows = 128
+        self.small_down_max_rows = 256 if H <= 1024 else 128
         # True folds each residual add + RMSNorm into the GEMM that consumes
         # its output (norm_linear_decode for q/k/v, norm_mlp_gate_lif for the
         # MLP): two launches fewer a layer, identical values, the residual
