@@ -743,8 +743,11 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(XDT == 
   // partition clamp to its last staged block (inside the cache; their words
   // are never used).  Called only when the wave has steps (nblk >= 1).  The
   // 2-wave kernel keeps slot_of: there the extra registers cost config 3
-  // 4.7 %.
-  const bool stride_blocks = KW == 4 && kStride >= (1 << p.bs_log2);
+  // 4.7 %, and so does head_dim 128, where the loop in both forms spilled 180
+  // bytes with five or more query heads a kv head (batch 256, ctx U[4096,
+  // 32768]: 384 -> 236 us without it, 5.1 TB/s; fixed 8k 199 -> 112 us).
+  constexpr bool kStrideBlocks = KW == 4 && W64 == 1;
+  const bool stride_blocks = kStrideBlocks && kStride >= (1 << p.bs_log2);
   const int lb4 = ((first + lo - start) >> p.bs_log2) * 4;  // byte offset in blocks[] at step 0
   const int sb4 = (kStride >> p.bs_log2) * 4;
   const int last4 = (nblk - 1) * 4;
@@ -781,7 +784,7 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(XDT == 
     });
   }
   };
-  if constexpr (KW == 4) {
+  if constexpr (kStrideBlocks) {
     if (stride_blocks) main_loop(std::true_type{});
     else main_loop(std::false_type{});
   } else {
