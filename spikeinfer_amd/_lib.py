@@ -165,6 +165,13 @@ def load(path: str | None = None) -> ctypes.CDLL:
     return lib
 
 
+# What csrc/native.cpp calls, in the order its bind() takes the addresses.
+NATIVE_FUNCTIONS = (
+    "spk_decode_attn", "spk_decode_attn_workspace_bytes", "spk_lif_pack_write_sites", "spk_lif_multistep",
+    "spk_prefill_attn", "spk_embed_rmsnorm", "spk_add_rmsnorm", "spk_rmsnorm_mean_t", "spk_lif_gate_mul",
+    "spk_linear_decode", "spk_mlp_gate_lif", "spk_qkv_rope_lif_pack_kv",
+)
+
 _UNBOUND = object()
 _native = _UNBOUND
 
@@ -181,11 +188,7 @@ def native():
         except ImportError:
             _native = None
         else:
-            mod.bind(*(ctypes.cast(getattr(lib, name), _vp).value for name in (
-                "spk_decode_attn", "spk_decode_attn_workspace_bytes", "spk_lif_pack_write_sites",
-                "spk_lif_multistep", "spk_prefill_attn", "spk_embed_rmsnorm", "spk_add_rmsnorm",
-                "spk_rmsnorm_mean_t", "spk_lif_gate_mul", "spk_linear_decode", "spk_mlp_gate_lif",
-                "spk_qkv_rope_lif_pack_kv")))
+            mod.bind("cuda", *(ctypes.cast(getattr(lib, name), _vp).value for name in NATIVE_FUNCTIONS))
             _native = mod
     return _native
 

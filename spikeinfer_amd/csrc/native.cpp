@@ -26,6 +26,10 @@
 
 namespace {
 
+// The kind of tensors taken: the GPU's, or the CPU's where the functions bound are
+// a test's stand-ins on the host.
+c10::DeviceType taken_on = at::kCUDA;
+
 decltype(&spk_decode_attn) decode_attn_fn;
 decltype(&spk_decode_attn_workspace_bytes) workspace_fn;
 decltype(&spk_lif_pack_write_sites) lif_sites_fn;
@@ -45,11 +49,12 @@ void need(bool ok) {
   if (!ok) throw NotTaken{};
 }
 
-// A plain tensor (no subclass, which may have its own semantics) on a GPU.
+// A plain tensor (no subclass, which may have its own semantics) on a GPU, with
+// memory of its own (torch.vmap's and torch.func's wrappers have none).
 const at::Tensor &tensor(PyObject *o) {
   need(THPVariable_CheckExact(o));
   const at::Tensor &t = THPVariable_Unpack(o);
-  need(t.device().type() == at::kCUDA && t.layout() == at::kStrided && !t.is_conj() && !t.is_neg());
+  need(t.device().type() == taken_on && t.layout() == at::kStrided && !t.is_conj() && !t.is_neg() && t.has_storage());
   return t;
 }
 
@@ -85,7 +90,9 @@ at::ScalarType dtype_of(PyObject *o) {
   return reinterpret_cast<THPDtype *>(o)->scalar_type;
 }
 
-void *stream_of(const at::Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+void *stream_of(const at::Tensor &t) {
+  return taken_on == at::kCUDA ? c10::hip::getCurrentHIPStream(t.device().index()).stream() : nullptr;
+}
 
 at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor &like) {
   return at::empty(sizes, at::TensorOptions().dtype(dtype).device(like.device()));
@@ -102,12 +109,24 @@ bool packed4(const at::Tensor &t) {
   return t.scalar_type() == at::kInt && t.dim() == 4 && t.stride(3) == 1;
 }
 
-// Runs a launch without the interpreter lock; a refused call is not taken (the
-// wrapper repeats it and raises its error).
-template <class F> void launch(F f) {
+// The interpreter lock, given up while an object of this type lives.
+struct Unlocked {
+  PyThreadState *const state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+template <class T> struct Same { typedef T type; };
+
+// Calls fn(args...) without the interpreter lock; the arguments, and whatever may
+// throw in working them out, are the caller's, before the lock is given up.  A
+// refused call is not taken (the wrapper repeats it and raises its error).
+template <class... P> void launch(int (*fn)(P...), typename Same<P>::type... args) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS rc = f();
-  Py_END_ALLOW_THREADS need(rc == SPK_OK);
+  {
+    const Unlocked unlocked;
+    rc = fn(args...);
+  }
+  need(rc == SPK_OK);
 }
 
 // Calls f, turning NotTaken and C++ errors (an allocation that fails) into None.
@@ -159,15 +178,13 @@ PyObject *decode_attn(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
     const Strides qs(q), ks(k), vs(v), os(out);
     void *const stream = stream_of(q);
-    launch([&] {
-      return decode_attn_fn(static_cast<const int32_t *>(q.data_ptr()), qs.s, static_cast<const int32_t *>(k.data_ptr()),
-                            ks.s, static_cast<const int32_t *>(v.data_ptr()), vs.s, k.size(2),
-                            static_cast<const int32_t *>(bt.data_ptr()), bt.stride(0), bt.stride(1),
-                            static_cast<const int32_t *>(lens.data_ptr()), out.data_ptr(), code, os.s,
-                            static_cast<int>(T), static_cast<int>(N), Hq, Hkv, D, bs, mb,
-                            static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))),
-                            bytes ? ws.data_ptr() : nullptr, bytes, stream);
-    });
+    launch(decode_attn_fn, static_cast<const int32_t *>(q.data_ptr()), qs.s, static_cast<const int32_t *>(k.data_ptr()),
+           ks.s, static_cast<const int32_t *>(v.data_ptr()), vs.s, k.size(2),
+           static_cast<const int32_t *>(bt.data_ptr()), bt.stride(0), bt.stride(1),
+           static_cast<const int32_t *>(lens.data_ptr()), out.data_ptr(), code, os.s,
+           static_cast<int>(T), static_cast<int>(N), Hq, Hkv, D, bs, mb,
+           static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))),
+           bytes ? ws.data_ptr() : nullptr, bytes, stream);
     if (a[9] != Py_None) return Py_NewRef(a[9]);
     return THPVariable_Wrap(out);
   });
@@ -227,10 +244,8 @@ PyObject *lif_sites(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
     void *const stream = stream_of(*first);
     const int T = static_cast<int>(first->size(0));
-    launch([&] {
-      return lif_sites_fn(sites, static_cast<int>(count), x_code, T,
-                          slots ? static_cast<const int64_t *>(slots->data_ptr()) : nullptr, stream);
-    });
+    launch(lif_sites_fn, sites, static_cast<int>(count), x_code, T,
+           slots ? static_cast<const int64_t *>(slots->data_ptr()) : nullptr, stream);
     Py_RETURN_TRUE;
   });
 }
@@ -253,11 +268,9 @@ PyObject *lif(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (membrane) u = empty(x.sizes().slice(1), at::kFloat, x);
     const int64_t strides[3] = {M * N, N, 1};
     void *const stream = stream_of(x);
-    launch([&] {
-      return lif_fn(x.data_ptr(), xc, strides, beta.data_ptr(), th.data_ptr(), pc, nullptr, spikes.data_ptr(), xc,
-                    membrane ? static_cast<float *>(u.data_ptr()) : nullptr, static_cast<int>(T), M,
-                    static_cast<int>(N), stream);
-    });
+    launch(lif_fn, x.data_ptr(), xc, strides, beta.data_ptr(), th.data_ptr(), pc, nullptr, spikes.data_ptr(), xc,
+           membrane ? static_cast<float *>(u.data_ptr()) : nullptr, static_cast<int>(T), M,
+           static_cast<int>(N), stream);
     if (!membrane) return THPVariable_Wrap(spikes);
     PyObject *r = PyTuple_New(2);
     need(r != nullptr);
@@ -310,12 +323,10 @@ PyObject *prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int code = float_code(out.scalar_type());
     char *const dst = static_cast<char *>(out.data_ptr()) + shift * out.stride(1) * out.element_size();
     void *const stream = stream_of(q);
-    launch([&] {
-      return prefill_fn(static_cast<const int32_t *>(q.data_ptr()), qs.s, static_cast<const int32_t *>(k.data_ptr()),
-                        static_cast<const int32_t *>(v.data_ptr()), ks.s, k.size(2), chunks, static_cast<int>(count),
-                        dst, code, os.s, static_cast<int>(T), static_cast<int>(Hq), static_cast<int>(k.size(1)), D, bs,
-                        static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))), stream);
-    });
+    launch(prefill_fn, static_cast<const int32_t *>(q.data_ptr()), qs.s, static_cast<const int32_t *>(k.data_ptr()),
+           static_cast<const int32_t *>(v.data_ptr()), ks.s, k.size(2), chunks, static_cast<int>(count),
+           dst, code, os.s, static_cast<int>(T), static_cast<int>(Hq), static_cast<int>(k.size(1)), D, bs,
+           static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))), stream);
     Py_RETURN_TRUE;
   });
 }
@@ -347,10 +358,8 @@ PyObject *embed_rmsnorm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     need(hidden < (1 << 30));
     const at::Tensor h = empty({T, rows, hidden}, embed.scalar_type(), embed), x = at::empty_like(h);
     void *const stream = stream_of(embed);
-    launch([&] {
-      return embed_fn(static_cast<const int64_t *>(ids.data_ptr()), embed.data_ptr(), embed.size(0), w.data_ptr(),
-                      h.data_ptr(), x.data_ptr(), code, T, rows, static_cast<int>(hidden), eps, stream);
-    });
+    launch(embed_fn, static_cast<const int64_t *>(ids.data_ptr()), embed.data_ptr(), embed.size(0), w.data_ptr(),
+           h.data_ptr(), x.data_ptr(), code, T, rows, static_cast<int>(hidden), eps, stream);
     PyObject *r = PyTuple_New(2);
     need(r != nullptr);
     PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(h));
@@ -376,10 +385,8 @@ PyObject *add_rmsnorm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     else out = alike(a[4], h);
     need(out.numel() == h.numel());
     void *const stream = stream_of(h);
-    launch([&] {
-      return add_norm_fn(h.data_ptr(), delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code,
-                         h.numel() / hidden, static_cast<int>(hidden), eps, stream);
-    });
+    launch(add_norm_fn, h.data_ptr(), delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code,
+           h.numel() / hidden, static_cast<int>(hidden), eps, stream);
     if (a[4] != Py_None) return Py_NewRef(a[4]);
     return THPVariable_Wrap(out);
   });
@@ -397,10 +404,8 @@ PyObject *rmsnorm_mean_t(PyObject *, PyObject *const *a, Py_ssize_t n) {
     need((!delta || delta->sizes() == h.sizes()) && w.numel() == h.size(2) && h.size(0) <= 8 && h.size(2) < (1 << 30));
     const at::Tensor out = empty({h.size(1), h.size(2)}, h.scalar_type(), h);
     void *const stream = stream_of(h);
-    launch([&] {
-      return mean_fn(h.data_ptr(), delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code,
-                     static_cast<int>(h.size(0)), h.size(1), static_cast<int>(h.size(2)), eps, stream);
-    });
+    launch(mean_fn, h.data_ptr(), delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code,
+           static_cast<int>(h.size(0)), h.size(1), static_cast<int>(h.size(2)), eps, stream);
     return THPVariable_Wrap(out);
   });
 }
@@ -418,10 +423,8 @@ PyObject *lif_gate_mul(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const at::Tensor out = empty({x.size(0), x.size(1), I}, x.scalar_type(), x);
     const int64_t strides[2] = {x.stride(0), x.stride(1)};
     void *const stream = stream_of(x);
-    launch([&] {
-      return gate_mul_fn(x.data_ptr(), code, strides, beta.data_ptr(), th.data_ptr(), pc, out.data_ptr(),
-                         static_cast<int>(x.size(0)), x.size(1), static_cast<int>(I), stream);
-    });
+    launch(gate_mul_fn, x.data_ptr(), code, strides, beta.data_ptr(), th.data_ptr(), pc, out.data_ptr(),
+           static_cast<int>(x.size(0)), x.size(1), static_cast<int>(I), stream);
     return THPVariable_Wrap(out);
   });
 }
@@ -446,10 +449,8 @@ PyObject *linear_decode(PyObject *, PyObject *const *a, Py_ssize_t n) {
       need(y.dim() >= 1 && y.size(-1) == N && y.numel() == M * N);
     }
     void *const stream = stream_of(x);
-    launch([&] {
-      return linear_fn(x.data_ptr(), w.data_ptr(), bias ? bias->data_ptr() : nullptr, y.data_ptr(),
-                       static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), SPK_BF16, stream);
-    });
+    launch(linear_fn, x.data_ptr(), w.data_ptr(), bias ? bias->data_ptr() : nullptr, y.data_ptr(),
+           static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), SPK_BF16, stream);
     if (a[3] != Py_None) return Py_NewRef(a[3]);
     return THPVariable_Wrap(y);
   });
@@ -469,11 +470,9 @@ PyObject *mlp_gate_lif(PyObject *, PyObject *const *a, Py_ssize_t n) {
          x.size(0) < (1 << 20) && x.size(1) < (1 << 28));
     const at::Tensor y = empty({x.size(0), x.size(1), I}, x.scalar_type(), x);
     void *const stream = stream_of(x);
-    launch([&] {
-      return mlp_gate_fn(x.data_ptr(), w.data_ptr(), beta.data_ptr(), th.data_ptr(), SPK_F32, y.data_ptr(),
-                         static_cast<int>(x.size(0)), static_cast<int>(x.size(1)), static_cast<int>(hidden),
-                         static_cast<int>(I), SPK_BF16, stream);
-    });
+    launch(mlp_gate_fn, x.data_ptr(), w.data_ptr(), beta.data_ptr(), th.data_ptr(), SPK_F32, y.data_ptr(),
+           static_cast<int>(x.size(0)), static_cast<int>(x.size(1)), static_cast<int>(hidden),
+           static_cast<int>(I), SPK_BF16, stream);
     return THPVariable_Wrap(y);
   });
 }
@@ -521,26 +520,27 @@ PyObject *qkv_rope_lif_pack(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int pc = float_code(beta.scalar_type());
     void *const stream = stream_of(x);
     auto words = [](const at::Tensor *t) { return t ? static_cast<int32_t *>(t->data_ptr()) : nullptr; };
-    launch([&] {
-      return qkv_fn(x.data_ptr(), code, xs, cos.data_ptr(), sin.data_ptr(),
-                    static_cast<const int64_t *>(pos.data_ptr()), cos.size(0), beta.data_ptr(), th.data_ptr(), pc,
-                    words(q), qs, n_q, words(&k), words(&v), cs, static_cast<const int64_t *>(slots.data_ptr()),
-                    k.size(2), words(own[0]), words(own[1]), nullptr, nullptr, nullptr, static_cast<int>(T), n_tok, Hq,
-                    Hkv, D, stream);
-    });
+    launch(qkv_fn, x.data_ptr(), code, xs, cos.data_ptr(), sin.data_ptr(),
+           static_cast<const int64_t *>(pos.data_ptr()), cos.size(0), beta.data_ptr(), th.data_ptr(), pc,
+           words(q), qs, n_q, words(&k), words(&v), cs, static_cast<const int64_t *>(slots.data_ptr()),
+           k.size(2), words(own[0]), words(own[1]), nullptr, nullptr, nullptr, static_cast<int>(T), n_tok, Hq,
+           Hkv, D, stream);
     Py_RETURN_TRUE;
   });
 }
 
 template <class F> void set(F &f, void *p) { f = reinterpret_cast<F>(p); }
 
-// bind(addresses): the C ABI's functions in the order of the declarations above.
+// bind(device, addresses): "cuda" or "cpu", and the C ABI's functions in the order of
+// the declarations above.
 PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
   constexpr int kFns = 12;
-  if (n != kFns) {
-    PyErr_Format(PyExc_TypeError, "bind takes %d addresses", kFns);
+  if (n != kFns + 1 || !PyUnicode_Check(a[0])) {
+    PyErr_Format(PyExc_TypeError, "bind takes a device type and %d addresses", kFns);
     return nullptr;
   }
+  taken_on = PyUnicode_CompareWithASCIIString(a[0], "cpu") == 0 ? at::kCPU : at::kCUDA;
+  ++a;
   void *p[kFns];
   for (int i = 0; i < kFns; ++i) {
     p[i] = PyLong_AsVoidPtr(a[i]);
