@@ -169,7 +169,7 @@ def load(path: str | None = None) -> ctypes.CDLL:
 NATIVE_FUNCTIONS = (
     "spk_decode_attn", "spk_decode_attn_workspace_bytes", "spk_lif_pack_write_sites", "spk_lif_multistep",
     "spk_prefill_attn", "spk_embed_rmsnorm", "spk_add_rmsnorm", "spk_rmsnorm_mean_t", "spk_lif_gate_mul",
-    "spk_linear_decode", "spk_mlp_gate_lif", "spk_qkv_rope_lif_pack_kv",
+    "spk_linear_decode", "spk_mlp_gate_lif", "spk_qkv_rope_lif_pack_kv", "spk_last_error",
 )
 
 _UNBOUND = object()

@@ -7,7 +7,10 @@
 // tensors on one GPU, already in the dtypes and layouts the C ABI takes -- and
 // returns None, with nothing launched, for every other form: the Python wrapper
 // then goes on as it would without this module, converting, or raising the error
-// the caller should see.  Nothing is kept between calls.
+// the caller should see.  An error that the library reports once it has come to
+// launching is raised here: the kernel may be queued, and an operator that updates
+// in place must not run twice.  Whatever else can fail comes before the launch.
+// Nothing is kept between calls.
 //
 // Calls reach the kernels through the C ABI (include/spikeinfer_amd.h) at the
 // addresses bind() is given, so one library is loaded, by _lib.py.  The
@@ -18,6 +21,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <cmath>
 #include <cstring>
@@ -42,9 +46,12 @@ decltype(&spk_lif_gate_mul) gate_mul_fn;
 decltype(&spk_linear_decode) linear_fn;
 decltype(&spk_mlp_gate_lif) mlp_gate_fn;
 decltype(&spk_qkv_rope_lif_pack_kv) qkv_fn;
+decltype(&spk_last_error) last_error_fn;
 
 // A call this module does not take (never seen by the caller).
 struct NotTaken {};
+// A call that failed with its Python exception set.
+struct Failed {};
 void need(bool ok) {
   if (!ok) throw NotTaken{};
 }
@@ -118,15 +125,33 @@ struct Unlocked {
 template <class T> struct Same { typedef T type; };
 
 // Calls fn(args...) without the interpreter lock; the arguments, and whatever may
-// throw in working them out, are the caller's, before the lock is given up.  A
-// refused call is not taken (the wrapper repeats it and raises its error).
-template <class... P> void launch(int (*fn)(P...), typename Same<P>::type... args) {
+// throw in working them out, are the caller's, before the lock is given up.
+// SPK_EINVAL and SPK_EUNSUPPORTED come before anything is launched: the call is
+// not taken, and the wrapper repeats it and raises its error.  SPK_EHIP is read
+// after a launch (and may be an earlier call's error): raised as _lib.check does.
+template <class... P> void launch(const char *what, int (*fn)(P...), typename Same<P>::type... args) {
   int rc;
   {
     const Unlocked unlocked;
     rc = fn(args...);
   }
-  need(rc == SPK_OK);
+  need(rc != SPK_EINVAL && rc != SPK_EUNSUPPORTED);
+  if (rc == SPK_OK) return;
+  PyErr_Format(PyExc_RuntimeError, "%s: %s", what, last_error_fn());
+  throw Failed{};
+}
+
+// What a call returns, made before its launch: the tensor given by the caller, or
+// the new one.
+THPObjectPtr result(PyObject *given, const at::Tensor &made) {
+  return THPObjectPtr(given == Py_None ? THPVariable_Wrap(made) : Py_NewRef(given));
+}
+THPObjectPtr pair(const at::Tensor &a, const at::Tensor &b) {
+  THPObjectPtr r(PyTuple_New(2));
+  need(r.get() != nullptr);
+  PyTuple_SET_ITEM(r.get(), 0, THPVariable_Wrap(a));
+  PyTuple_SET_ITEM(r.get(), 1, THPVariable_Wrap(b));
+  return r;
 }
 
 // Calls f, turning NotTaken and C++ errors (an allocation that fails) into None.
@@ -134,6 +159,8 @@ template <class F> PyObject *guarded(Py_ssize_t given, Py_ssize_t wanted, F f) {
   try {
     need(given == wanted && !c10::impl::dispatch_mode_enabled());
     return f();
+  } catch (const Failed &) {
+    return nullptr;
   } catch (const NotTaken &) {
   } catch (const std::exception &) {
   }
@@ -178,15 +205,14 @@ PyObject *decode_attn(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
     const Strides qs(q), ks(k), vs(v), os(out);
     void *const stream = stream_of(q);
-    launch(decode_attn_fn, static_cast<const int32_t *>(q.data_ptr()), qs.s, static_cast<const int32_t *>(k.data_ptr()),
-           ks.s, static_cast<const int32_t *>(v.data_ptr()), vs.s, k.size(2),
-           static_cast<const int32_t *>(bt.data_ptr()), bt.stride(0), bt.stride(1),
-           static_cast<const int32_t *>(lens.data_ptr()), out.data_ptr(), code, os.s,
-           static_cast<int>(T), static_cast<int>(N), Hq, Hkv, D, bs, mb,
-           static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))),
+    THPObjectPtr done = result(a[9], out);
+    launch("paged_spike_attn_decode", decode_attn_fn, static_cast<const int32_t *>(q.data_ptr()), qs.s,
+           static_cast<const int32_t *>(k.data_ptr()), ks.s, static_cast<const int32_t *>(v.data_ptr()), vs.s,
+           k.size(2), static_cast<const int32_t *>(bt.data_ptr()), bt.stride(0), bt.stride(1),
+           static_cast<const int32_t *>(lens.data_ptr()), out.data_ptr(), code, os.s, static_cast<int>(T),
+           static_cast<int>(N), Hq, Hkv, D, bs, mb, static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))),
            bytes ? ws.data_ptr() : nullptr, bytes, stream);
-    if (a[9] != Py_None) return Py_NewRef(a[9]);
-    return THPVariable_Wrap(out);
+    return done.release();
   });
 }
 
@@ -244,7 +270,7 @@ PyObject *lif_sites(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
     void *const stream = stream_of(*first);
     const int T = static_cast<int>(first->size(0));
-    launch(lif_sites_fn, sites, static_cast<int>(count), x_code, T,
+    launch("lif_pack_write_sites", lif_sites_fn, sites, static_cast<int>(count), x_code, T,
            slots ? static_cast<const int64_t *>(slots->data_ptr()) : nullptr, stream);
     Py_RETURN_TRUE;
   });
@@ -268,15 +294,11 @@ PyObject *lif(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (membrane) u = empty(x.sizes().slice(1), at::kFloat, x);
     const int64_t strides[3] = {M * N, N, 1};
     void *const stream = stream_of(x);
-    launch(lif_fn, x.data_ptr(), xc, strides, beta.data_ptr(), th.data_ptr(), pc, nullptr, spikes.data_ptr(), xc,
-           membrane ? static_cast<float *>(u.data_ptr()) : nullptr, static_cast<int>(T), M,
+    THPObjectPtr done = membrane ? pair(spikes, u) : result(Py_None, spikes);
+    launch("lif_multistep", lif_fn, x.data_ptr(), xc, strides, beta.data_ptr(), th.data_ptr(), pc, nullptr,
+           spikes.data_ptr(), xc, membrane ? static_cast<float *>(u.data_ptr()) : nullptr, static_cast<int>(T), M,
            static_cast<int>(N), stream);
-    if (!membrane) return THPVariable_Wrap(spikes);
-    PyObject *r = PyTuple_New(2);
-    need(r != nullptr);
-    PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(spikes));
-    PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(u));
-    return r;
+    return done.release();
   });
 }
 
@@ -323,10 +345,10 @@ PyObject *prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int code = float_code(out.scalar_type());
     char *const dst = static_cast<char *>(out.data_ptr()) + shift * out.stride(1) * out.element_size();
     void *const stream = stream_of(q);
-    launch(prefill_fn, static_cast<const int32_t *>(q.data_ptr()), qs.s, static_cast<const int32_t *>(k.data_ptr()),
-           static_cast<const int32_t *>(v.data_ptr()), ks.s, k.size(2), chunks, static_cast<int>(count),
-           dst, code, os.s, static_cast<int>(T), static_cast<int>(Hq), static_cast<int>(k.size(1)), D, bs,
-           static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))), stream);
+    launch("paged_spike_attn_prefill", prefill_fn, static_cast<const int32_t *>(q.data_ptr()), qs.s,
+           static_cast<const int32_t *>(k.data_ptr()), static_cast<const int32_t *>(v.data_ptr()), ks.s, k.size(2),
+           chunks, static_cast<int>(count), dst, code, os.s, static_cast<int>(T), static_cast<int>(Hq),
+           static_cast<int>(k.size(1)), D, bs, static_cast<float>(1.0 / std::sqrt(static_cast<double>(D))), stream);
     Py_RETURN_TRUE;
   });
 }
@@ -358,13 +380,10 @@ PyObject *embed_rmsnorm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     need(hidden < (1 << 30));
     const at::Tensor h = empty({T, rows, hidden}, embed.scalar_type(), embed), x = at::empty_like(h);
     void *const stream = stream_of(embed);
-    launch(embed_fn, static_cast<const int64_t *>(ids.data_ptr()), embed.data_ptr(), embed.size(0), w.data_ptr(),
-           h.data_ptr(), x.data_ptr(), code, T, rows, static_cast<int>(hidden), eps, stream);
-    PyObject *r = PyTuple_New(2);
-    need(r != nullptr);
-    PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(h));
-    PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(x));
-    return r;
+    THPObjectPtr done = pair(h, x);
+    launch("embed_rmsnorm", embed_fn, static_cast<const int64_t *>(ids.data_ptr()), embed.data_ptr(), embed.size(0),
+           w.data_ptr(), h.data_ptr(), x.data_ptr(), code, T, rows, static_cast<int>(hidden), eps, stream);
+    return done.release();
   });
 }
 
@@ -385,10 +404,10 @@ PyObject *add_rmsnorm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     else out = alike(a[4], h);
     need(out.numel() == h.numel());
     void *const stream = stream_of(h);
-    launch(add_norm_fn, h.data_ptr(), delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code,
-           h.numel() / hidden, static_cast<int>(hidden), eps, stream);
-    if (a[4] != Py_None) return Py_NewRef(a[4]);
-    return THPVariable_Wrap(out);
+    THPObjectPtr done = result(a[4], out);
+    launch("add_rmsnorm", add_norm_fn, h.data_ptr(),
+           delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code, h.numel() / hidden, static_cast<int>(hidden), eps, stream);
+    return done.release();
   });
 }
 
@@ -404,9 +423,10 @@ PyObject *rmsnorm_mean_t(PyObject *, PyObject *const *a, Py_ssize_t n) {
     need((!delta || delta->sizes() == h.sizes()) && w.numel() == h.size(2) && h.size(0) <= 8 && h.size(2) < (1 << 30));
     const at::Tensor out = empty({h.size(1), h.size(2)}, h.scalar_type(), h);
     void *const stream = stream_of(h);
-    launch(mean_fn, h.data_ptr(), delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code,
-           static_cast<int>(h.size(0)), h.size(1), static_cast<int>(h.size(2)), eps, stream);
-    return THPVariable_Wrap(out);
+    THPObjectPtr done = result(Py_None, out);
+    launch("rmsnorm_mean_t", mean_fn, h.data_ptr(),
+           delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code, static_cast<int>(h.size(0)), h.size(1), static_cast<int>(h.size(2)), eps, stream);
+    return done.release();
   });
 }
 
@@ -423,9 +443,10 @@ PyObject *lif_gate_mul(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const at::Tensor out = empty({x.size(0), x.size(1), I}, x.scalar_type(), x);
     const int64_t strides[2] = {x.stride(0), x.stride(1)};
     void *const stream = stream_of(x);
-    launch(gate_mul_fn, x.data_ptr(), code, strides, beta.data_ptr(), th.data_ptr(), pc, out.data_ptr(),
+    THPObjectPtr done = result(Py_None, out);
+    launch("lif_gate_mul", gate_mul_fn, x.data_ptr(), code, strides, beta.data_ptr(), th.data_ptr(), pc, out.data_ptr(),
            static_cast<int>(x.size(0)), x.size(1), static_cast<int>(I), stream);
-    return THPVariable_Wrap(out);
+    return done.release();
   });
 }
 
@@ -449,10 +470,10 @@ PyObject *linear_decode(PyObject *, PyObject *const *a, Py_ssize_t n) {
       need(y.dim() >= 1 && y.size(-1) == N && y.numel() == M * N);
     }
     void *const stream = stream_of(x);
-    launch(linear_fn, x.data_ptr(), w.data_ptr(), bias ? bias->data_ptr() : nullptr, y.data_ptr(),
-           static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), SPK_BF16, stream);
-    if (a[3] != Py_None) return Py_NewRef(a[3]);
-    return THPVariable_Wrap(y);
+    THPObjectPtr done = result(a[3], y);
+    launch("linear_decode", linear_fn, x.data_ptr(), w.data_ptr(),
+           bias ? bias->data_ptr() : nullptr, y.data_ptr(), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), SPK_BF16, stream);
+    return done.release();
   });
 }
 
@@ -470,10 +491,11 @@ PyObject *mlp_gate_lif(PyObject *, PyObject *const *a, Py_ssize_t n) {
          x.size(0) < (1 << 20) && x.size(1) < (1 << 28));
     const at::Tensor y = empty({x.size(0), x.size(1), I}, x.scalar_type(), x);
     void *const stream = stream_of(x);
-    launch(mlp_gate_fn, x.data_ptr(), w.data_ptr(), beta.data_ptr(), th.data_ptr(), SPK_F32, y.data_ptr(),
-           static_cast<int>(x.size(0)), static_cast<int>(x.size(1)), static_cast<int>(hidden),
+    THPObjectPtr done = result(Py_None, y);
+    launch("mlp_gate_lif", mlp_gate_fn, x.data_ptr(), w.data_ptr(), beta.data_ptr(), th.data_ptr(), SPK_F32,
+           y.data_ptr(), static_cast<int>(x.size(0)), static_cast<int>(x.size(1)), static_cast<int>(hidden),
            static_cast<int>(I), SPK_BF16, stream);
-    return THPVariable_Wrap(y);
+    return done.release();
   });
 }
 
@@ -520,11 +542,10 @@ PyObject *qkv_rope_lif_pack(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int pc = float_code(beta.scalar_type());
     void *const stream = stream_of(x);
     auto words = [](const at::Tensor *t) { return t ? static_cast<int32_t *>(t->data_ptr()) : nullptr; };
-    launch(qkv_fn, x.data_ptr(), code, xs, cos.data_ptr(), sin.data_ptr(),
-           static_cast<const int64_t *>(pos.data_ptr()), cos.size(0), beta.data_ptr(), th.data_ptr(), pc,
-           words(q), qs, n_q, words(&k), words(&v), cs, static_cast<const int64_t *>(slots.data_ptr()),
-           k.size(2), words(own[0]), words(own[1]), nullptr, nullptr, nullptr, static_cast<int>(T), n_tok, Hq,
-           Hkv, D, stream);
+    launch("qkv_rope_lif_pack", qkv_fn, x.data_ptr(), code, xs, cos.data_ptr(), sin.data_ptr(),
+           static_cast<const int64_t *>(pos.data_ptr()), cos.size(0), beta.data_ptr(), th.data_ptr(), pc, words(q), qs,
+           n_q, words(&k), words(&v), cs, static_cast<const int64_t *>(slots.data_ptr()), k.size(2), words(own[0]),
+           words(own[1]), nullptr, nullptr, nullptr, static_cast<int>(T), n_tok, Hq, Hkv, D, stream);
     Py_RETURN_TRUE;
   });
 }
@@ -534,7 +555,7 @@ template <class F> void set(F &f, void *p) { f = reinterpret_cast<F>(p); }
 // bind(device, addresses): "cuda" or "cpu", and the C ABI's functions in the order of
 // the declarations above.
 PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
-  constexpr int kFns = 12;
+  constexpr int kFns = 13;
   if (n != kFns + 1 || !PyUnicode_Check(a[0])) {
     PyErr_Format(PyExc_TypeError, "bind takes a device type and %d addresses", kFns);
     return nullptr;
@@ -561,6 +582,7 @@ PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
   set(linear_fn, p[9]);
   set(mlp_gate_fn, p[10]);
   set(qkv_fn, p[11]);
+  set(last_error_fn, p[12]);
   Py_RETURN_NONE;
 }
 

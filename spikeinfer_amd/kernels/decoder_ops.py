@@ -13,7 +13,7 @@ import torch
 from .. import _lib
 
 # Each operator first offers its arguments to the C++ entry (csrc/native.cpp),
-# which takes their usual form and answers None, having done nothing, otherwise.
+# which takes their usual form and answers None, having launched nothing, otherwise.
 
 _VEC_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 

@@ -17,6 +17,7 @@ from spikeinfer_amd import _lib
 from spikeinfer_amd.build import NATIVE_PATH
 
 
+ERROR = ctypes.create_string_buffer(b"the stand-in's error")
 bound = {}  # module file -> its stand-ins, which it calls as long as it lives
 
 
@@ -33,7 +34,10 @@ def load_with_stubs(folder, **stubs):
         # (pointers as plain addresses: a callback gets no typed pointer from C)
         args = [ctypes.c_void_p if a not in (ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_size_t) else a
                 for a in args]
-        fn = ctypes.CFUNCTYPE(res, *args)(stubs.get(name, lambda *a: 0))
+        default = lambda *a: 0
+        if name == "spk_last_error":
+            res, default = ctypes.c_void_p, lambda: ctypes.addressof(ERROR)
+        fn = ctypes.CFUNCTYPE(res, *args)(stubs.get(name, default))
         keep.append(fn)
         addresses.append(ctypes.cast(fn, ctypes.c_void_p).value)
     mod.bind("cpu", *addresses)
@@ -82,3 +86,68 @@ def test_the_interpreter_is_free_during_a_launch(tmp_path):
     for t in threads:
         t.join(120)
     assert all(g is not None and g.shape == (4, 3, 8) for g in got)
+
+
+def _calls(n=64):
+    """Each operator's name in the module, its C function and arguments it takes."""
+    f, b16 = torch.float32, torch.bfloat16
+    z = lambda *s, dt=f: torch.zeros(s, dtype=dt)
+    i32, i64 = torch.int32, torch.int64
+    q, kv = z(4, 2, 4, 2, dt=i32), z(4, 2, 32, 2, dt=i32)
+    lens, table = torch.ones(2, dtype=i32), z(2, 2, dt=i32)
+    h, w = z(4, 3, n, dt=b16), z(n, dt=b16)
+    qkv, rope = z(4, 2, 8 * 64, dt=b16), z(5, 64, dt=b16)
+    slots = torch.arange(2)
+    return [
+        ("decode_attn", "spk_decode_attn", (q, kv, kv, table, lens, 64, 16, 4, 2, None, f, None)),
+        ("lif_sites", "spk_lif_pack_write_sites", ([(z(4, 2, 4, 64), z(64), z(64), q, False)], None)),
+        ("lif", "spk_lif_multistep", (z(4, 3, n), z(n), z(n), True)),
+        ("prefill", "spk_prefill_attn", (q, kv, kv, [(0, 0, 2, 1, table[0])], z(4, 2, 4, 64), 64, 16)),
+        ("embed_rmsnorm", "spk_embed_rmsnorm", (z(3, dt=i64), z(9, n, dt=b16), w, 1e-6, 4)),
+        ("add_rmsnorm", "spk_add_rmsnorm", (h, torch.ones_like(h), w, 1e-6, None)),
+        ("rmsnorm_mean_t", "spk_rmsnorm_mean_t", (h, w, 1e-6, None)),
+        ("lif_gate_mul", "spk_lif_gate_mul", (h, z(n // 2), z(n // 2))),
+        ("linear_decode", "spk_linear_decode", (h, z(16, n, dt=b16), None, None)),
+        ("mlp_gate_lif", "spk_mlp_gate_lif", (h, z(2 * 32, n, dt=b16), z(32), z(32))),
+        ("qkv_rope_lif_pack", "spk_qkv_rope_lif_pack_kv", (qkv, rope, rope, z(3, 64), z(3, 64), kv, kv, slots, 4, 2,
+                                                           64, q, 2, slots, None, None)),
+    ]
+
+
+@pytest.mark.parametrize("status", [_lib.SPK_OK, _lib.SPK_EINVAL, _lib.SPK_EUNSUPPORTED, _lib.SPK_EHIP])
+def test_a_call_is_repeated_only_if_nothing_was_launched(tmp_path, status):
+    """Refusals (decided before a launch) go back to the wrapper; an error read after
+    the launch is raised, so that nothing runs twice."""
+    for name, fn, args in _calls():
+        (tmp_path / name).mkdir()
+        seen = []
+        mod = load_with_stubs(tmp_path / name, **{fn: lambda *a: seen.append(a) or status})
+        call = getattr(mod, name)
+        if status == _lib.SPK_EHIP:
+            with pytest.raises(RuntimeError, match="the stand-in's error"):
+                call(*args)
+        else:
+            assert (call(*args) is None) == (status != _lib.SPK_OK), name
+        assert len(seen) == 1, name
+
+
+def test_the_residual_is_added_once(tmp_path, monkeypatch):
+    """add_rmsnorm updates h in place: through the wrapper, an error that is read
+    after the launch leaves one launch behind it and reaches the caller."""
+    from spikeinfer_amd.kernels.decoder_ops import add_rmsnorm
+
+    h, delta = torch.zeros(2, 8), torch.ones(2, 8)
+    seen = []
+
+    def launched(*a):
+        seen.append(h.add_(delta))
+        return _lib.SPK_EHIP if len(seen) == 1 else _lib.SPK_OK
+
+    monkeypatch.setattr(_lib, "_native", load_with_stubs(tmp_path, spk_add_rmsnorm=launched))
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t: torch.device("cpu"))
+    monkeypatch.setattr(_lib, "stream_of", lambda d: 0)
+    host = type("Host", (), {"spk_add_rmsnorm": staticmethod(launched)})
+    monkeypatch.setattr(_lib, "load", lambda path=None: host)
+    with pytest.raises(RuntimeError, match="add_rmsnorm: the stand-in's error"):
+        add_rmsnorm(h, delta, torch.ones(8), 1e-6)
+    assert len(seen) == 1 and torch.equal(h, delta)
