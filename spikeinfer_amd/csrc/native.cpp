@@ -328,7 +328,9 @@ PyObject *prefill(PyObject *, PyObject *const *a, Py_ssize_t n) {
       s.start = q_row;
       s.q_len = int32(PyTuple_GET_ITEM(c, 2));
       s.ctx = int32(PyTuple_GET_ITEM(c, 3));
-      need(s.q_len > 0 && q_row >= 0 && q_row + s.q_len <= q.size(1) && out_row >= 0 && out_row + s.q_len <= out.size(1));
+      // (differences of what lies in a tensor's range: a sum could pass 64 bits)
+      need(s.q_len > 0 && q_row >= 0 && q_row <= q.size(1) - s.q_len && out_row >= 0 &&
+           out_row <= out.size(1) - s.q_len);
       if (i == 0) shift = out_row - q_row;
       need(shift == out_row - q_row);
       PyObject *table = PyTuple_GET_ITEM(c, 4);
@@ -406,7 +408,8 @@ PyObject *add_rmsnorm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     void *const stream = stream_of(h);
     THPObjectPtr done = result(a[4], out);
     launch("add_rmsnorm", add_norm_fn, h.data_ptr(),
-           delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code, h.numel() / hidden, static_cast<int>(hidden), eps, stream);
+           delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code, h.numel() / hidden,
+           static_cast<int>(hidden), eps, stream);
     return done.release();
   });
 }
@@ -425,7 +428,8 @@ PyObject *rmsnorm_mean_t(PyObject *, PyObject *const *a, Py_ssize_t n) {
     void *const stream = stream_of(h);
     THPObjectPtr done = result(Py_None, out);
     launch("rmsnorm_mean_t", mean_fn, h.data_ptr(),
-           delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code, static_cast<int>(h.size(0)), h.size(1), static_cast<int>(h.size(2)), eps, stream);
+           delta ? delta->data_ptr() : nullptr, w.data_ptr(), out.data_ptr(), code, static_cast<int>(h.size(0)),
+           h.size(1), static_cast<int>(h.size(2)), eps, stream);
     return done.release();
   });
 }
@@ -472,7 +476,8 @@ PyObject *linear_decode(PyObject *, PyObject *const *a, Py_ssize_t n) {
     void *const stream = stream_of(x);
     THPObjectPtr done = result(a[3], y);
     launch("linear_decode", linear_fn, x.data_ptr(), w.data_ptr(),
-           bias ? bias->data_ptr() : nullptr, y.data_ptr(), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), SPK_BF16, stream);
+           bias ? bias->data_ptr() : nullptr, y.data_ptr(), static_cast<int>(M),
+           static_cast<int>(N), static_cast<int>(K), SPK_BF16, stream);
     return done.release();
   });
 }

@@ -151,3 +151,15 @@ def test_the_residual_is_added_once(tmp_path, monkeypatch):
     with pytest.raises(RuntimeError, match="add_rmsnorm: the stand-in's error"):
         add_rmsnorm(h, delta, torch.ones(8), 1e-6)
     assert len(seen) == 1 and torch.equal(h, delta)
+
+
+def test_rows_past_64_bits_are_not_taken(tmp_path):
+    """A chunk's first row near 2**63: the row after its last must not wrap round to
+    one inside the tensor."""
+    seen = []
+    mod = load_with_stubs(tmp_path, spk_prefill_attn=lambda *a: seen.append(a) or 0)
+    args = dict((name, a) for name, _, a in _calls())["prefill"]
+    for q_row, out_row in ((2**63 - 1, 0), (2**63 - 2, 2**63 - 2), (0, 2**63 - 1), (-1, 0), (1, 0), (0, 1)):
+        assert mod.prefill(*args[:3], [(q_row, out_row, 2, 0, args[3][0][4])], *args[4:]) is None
+    assert not seen
+    assert mod.prefill(*args) is True and len(seen) == 1
