@@ -443,7 +443,7 @@ extern "C" int spk_prefill_attn(const int32_t *q, const int64_t q_strides[3], co
     const int64_t rows = static_cast<int64_t>(c.q_len) * nrep;
     if (rows > (1 << 28) || rows * nrep > 0xffffffffll || static_cast<int64_t>(c.q_len) + c.ctx > (1 << 30))
       return fail(SPK_EUNSUPPORTED, "prefill_attn: chunk %d of %d + %d tokens is too long", i, c.ctx, c.q_len);
-    if (!c.table && c.start + c.q_len > num_slots)
+    if (!c.table && c.start > num_slots - c.q_len)
       return fail(SPK_EINVAL, "prefill_attn: chunk %d reaches past %lld slots", i, (long long)num_slots);
     total += static_cast<int64_t>(c.q_len) * nrep;
   }

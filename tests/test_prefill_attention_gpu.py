@@ -166,6 +166,7 @@ def test_bad_chunks_are_refused_on_the_host():
     assert call(pack(), dt=_lib.SPK_I32) == _lib.SPK_EINVAL
     assert call(pack(ctx=3)) == _lib.SPK_EINVAL       # cached prefix without a table
     assert call(pack(start=97)) == _lib.SPK_EINVAL    # past the slots
+    assert call(pack(start=2**63 - 2)) == _lib.SPK_EINVAL  # (the end past 64 bits)
     assert call(pack(q_len=-1)) == _lib.SPK_EINVAL
     assert call(pack(), n=0) == _lib.SPK_OK
     assert call(pack(q_len=0)) == _lib.SPK_OK         # nothing to do, nothing launched
