@@ -49,7 +49,10 @@ enum spk_dtype {
 /* Message of the last failing call on this thread ("" if none). */
 const char *spk_last_error(void);
 
-/* ABI version, bumped on any signature change (2: spk_decode_advance draws; 3: spk_decode_attn_combine takes the partials size, spk_norm_* GEMMs). */
+/* ABI version, bumped on any signature change and any new entry point (2: spk_decode_advance
+ * draws; 3: spk_decode_attn_combine takes the partials size, spk_norm_* GEMMs; 4: spk_prefill_attn,
+ * spk_qkv_rope_lif_pack_kv). */
+#define SPK_ABI_VERSION 4
 int spk_abi_version(void);
 
 /*

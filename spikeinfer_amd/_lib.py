@@ -29,7 +29,7 @@ _DTYPE_CODES = {
     torch.int32: SPK_I32,
 }
 
-ABI_VERSION = 3
+ABI_VERSION = 4  # SPK_ABI_VERSION
 DECODE_ATTN_SCRATCH_BYTES = 16 << 20  # SPK_DECODE_ATTN_SCRATCH_BYTES
 
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -152,14 +152,15 @@ def load(path: str | None = None) -> ctypes.CDLL:
             f"{path} not found: build it with `python -m spikeinfer_amd.build`"
         )
     lib = ctypes.CDLL(path)
-    for name, (res, args) in _SIGNATURES.items():
-        fn = getattr(lib, name)
-        fn.restype = res
-        fn.argtypes = args
+    # the version first: a library of another one may lack entry points
     if lib.spk_abi_version() != ABI_VERSION:
         raise RuntimeError(
             f"{path} has ABI {lib.spk_abi_version()}, expected {ABI_VERSION}: rebuild it"
         )
+    for name, (res, args) in _SIGNATURES.items():
+        fn = getattr(lib, name)
+        fn.restype = res
+        fn.argtypes = args
     if path == LIB_PATH:
         _lib = lib
     return lib

@@ -5,6 +5,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 import torch
@@ -28,6 +29,21 @@ def test_library_exports_every_declared_symbol():
     for name in _declared():
         assert hasattr(lib, name), name
     assert lib.spk_abi_version() == _lib.ABI_VERSION
+
+
+def test_a_library_of_another_version_is_named_as_such(tmp_path):
+    """An older library lacks entry points too: the version is looked at first, so
+    the error says to rebuild, not which symbol is missing."""
+    so = str(tmp_path / "old.so")
+    (tmp_path / "old.c").write_text("int spk_abi_version(void) { return 3; }")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", so, str(tmp_path / "old.c")], check=True)
+    with pytest.raises(RuntimeError, match="ABI 3, expected .*rebuild"):
+        _lib.load(so)
+
+
+def test_the_header_names_the_version():
+    text = open(HEADER).read()
+    assert re.search(rf"#define SPK_ABI_VERSION {_lib.ABI_VERSION}\b", text)
 
 
 def _i64(*v):
