@@ -179,18 +179,21 @@ _native = _UNBOUND
 
 def native():
     """The Python entry module (csrc/native.cpp) bound to the loaded library, or
-    None where it is not built for this torch: the wrappers' own path then
-    makes the same calls through ctypes."""
+    None where it is not built, or not for this C ABI and this torch: the
+    wrappers' own path then makes the same calls through ctypes."""
     global _native
     if _native is _UNBOUND:
         lib = load()
         try:
             from . import _native as mod
         except ImportError:
-            _native = None
-        else:
+            mod = None
+        built_for = (getattr(mod, "abi_version", None), getattr(mod, "built_for", None))
+        if built_for == (ABI_VERSION, torch.__version__):
             mod.bind("cuda", *(ctypes.cast(getattr(lib, name), _vp).value for name in NATIVE_FUNCTIONS))
             _native = mod
+        else:
+            _native = None
     return _native
 
 

@@ -603,4 +603,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }
+// The module carries what it was compiled for: the addresses that bind() takes are
+// called by this version of the C ABI, and tensors are read by this torch's layout.
+PyMODINIT_FUNC PyInit__native() {
+  THPObjectPtr m(PyModule_Create(&module));
+  if (!m || PyModule_AddIntConstant(m.get(), "abi_version", SPK_ABI_VERSION) ||
+      PyModule_AddStringConstant(m.get(), "built_for", SPK_TORCH_VERSION))
+    return nullptr;
+  return m.release();
+}

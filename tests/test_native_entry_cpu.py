@@ -4,15 +4,18 @@ that what happens around a launch can be looked at without one."""
 from __future__ import annotations
 
 import ctypes
+import importlib
 import importlib.util
 import shutil
 import subprocess
 import sys
 import threading
+import types
 
 import pytest
 import torch
 
+import spikeinfer_amd
 from spikeinfer_amd import _lib
 from spikeinfer_amd.build import NATIVE_PATH
 
@@ -163,3 +166,33 @@ def test_rows_past_64_bits_are_not_taken(tmp_path):
         assert mod.prefill(*args[:3], [(q_row, out_row, 2, 0, args[3][0][4])], *args[4:]) is None
     assert not seen
     assert mod.prefill(*args) is True and len(seen) == 1
+
+
+def _fresh(monkeypatch, module):
+    """_lib.native() as a new process would answer it with `module` beside it."""
+    monkeypatch.setattr(_lib, "_native", _lib._UNBOUND)
+    monkeypatch.setitem(sys.modules, "spikeinfer_amd._native", module)
+    monkeypatch.setattr(spikeinfer_amd, "_native", module, raising=False)
+    return _lib.native()
+
+
+def test_a_module_built_for_something_else_is_not_used(monkeypatch):
+    """Its calls go to bare addresses: another version of the C ABI or of torch
+    than it was compiled for means the wrappers' own path."""
+    binds = []
+    stamp = dict(abi_version=_lib.ABI_VERSION, built_for=torch.__version__)
+    for change, used in ((dict(), True), (dict(abi_version=3), False), (dict(built_for="2.0.0"), False),
+                         (dict(abi_version=None, built_for=None), False)):
+        mod = types.ModuleType("_native")
+        mod.bind = lambda *a: binds.append(a)
+        for name, value in {**stamp, **change}.items():
+            if value is not None:
+                setattr(mod, name, value)
+        assert _fresh(monkeypatch, mod) is (mod if used else None), change
+    assert len(binds) == 1
+
+
+def test_the_built_module_is_stamped_and_used(monkeypatch):
+    mod = importlib.import_module("spikeinfer_amd._native")
+    assert (mod.abi_version, mod.built_for) == (_lib.ABI_VERSION, torch.__version__)
+    assert _fresh(monkeypatch, mod) is mod
