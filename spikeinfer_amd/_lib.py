@@ -183,7 +183,10 @@ def native():
     wrappers' own path then makes the same calls through ctypes."""
     global _native
     if _native is _UNBOUND:
-        lib = load()
+        try:
+            lib = load()
+        except KernelLibraryMissing:  # raised by the wrapper's own load, after its checks
+            return None
         try:
             from . import _native as mod
         except ImportError:

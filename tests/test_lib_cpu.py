@@ -245,3 +245,30 @@ def test_norm_gemms_validate_on_the_host():
     assert lib.spk_norm_linear_decode(A, A, A, None, 1e-6, A, None, A, 64, 1152, 1280, bf16, None) == _lib.SPK_EUNSUPPORTED
     assert lib.spk_norm_mlp_gate_lif(A, A + 16, A, A, 1e-6, A, A, A, f32, A, 4, 8, 896, 4864, bf16, None) == _lib.SPK_EINVAL
     assert lib.spk_norm_mlp_gate_lif(None, A, A, None, 1e-6, A, A, A, f32, A, 4, 8, 896, 4864, bf16, None) == _lib.SPK_EINVAL
+
+
+def test_arguments_are_refused_without_the_library_too(monkeypatch, tmp_path):
+    """Bad arguments end in their own error where the library is not built; only a
+    call that would launch says that it is missing."""
+    from spikeinfer_amd.kernels import lif_multistep, paged_spike_attn_decode
+    from spikeinfer_amd.kernels.decoder_ops import add_rmsnorm, linear_decode
+    from spikeinfer_amd.kernels.spike_attention import paged_spike_attn_prefill
+
+    monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "absent.so"))
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "_native", _lib._UNBOUND)
+    x, p = torch.ones(4, 2, 64), torch.ones(64)
+    with pytest.raises(AssertionError, match="trailing dim"):
+        lif_multistep(x, p[:32], p)
+    for call in (lambda: lif_multistep(x, p, p), lambda: add_rmsnorm(x, None, p, 1e-6),
+                 lambda: linear_decode(x, torch.ones(16, 64)),
+                 lambda: paged_spike_attn_prefill(torch.zeros(4, 1, 2, 2, dtype=torch.int32), x, x, [], x, 64, 16)):
+        with pytest.raises(ValueError, match="GPU"):
+            call()
+    q = torch.zeros(4, 1, 14, 2, dtype=torch.int32)
+    with pytest.raises(ValueError, match="expected 1"):
+        paged_spike_attn_decode(q, q, q, q, q, 32, 16, 14, 2)
+    assert _lib._native is _lib._UNBOUND  # (looked for again once the library is there)
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t: torch.device("cpu"))
+    with pytest.raises(_lib.KernelLibraryMissing, match="build it"):
+        add_rmsnorm(x, None, p, 1e-6)
