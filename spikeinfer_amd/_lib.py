@@ -185,8 +185,8 @@ def native():
     if _native is _UNBOUND:
         try:
             lib = load()
-        except KernelLibraryMissing:  # raised by the wrapper's own load, after its checks
-            return None
+        except (RuntimeError, OSError):  # missing, another version, not loadable: raised by the
+            return None  # wrapper's own load, after its checks
         try:
             from . import _native as mod
         except ImportError:
