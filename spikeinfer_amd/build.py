@@ -64,25 +64,41 @@ def _run(cmd: list[str], verbose: bool) -> None:
         raise RuntimeError(f"{os.path.basename(cmd[0])} failed ({res.returncode}):\n{res.stderr}")
 
 
+def build_native(verbose: bool = False) -> str | None:
+    """Compiles csrc/native.cpp into the Python entry module; what failed, if it
+    did (an older module is then removed: it may be of another C ABI)."""
+    tmp = NATIVE_PATH + ".tmp"
+    try:
+        _run(native_command(tmp), verbose)
+        os.replace(tmp, NATIVE_PATH)
+        return None
+    except Exception as e:  # no compiler, no headers of torch or Python, a compile error
+        if os.path.exists(NATIVE_PATH):
+            os.remove(NATIVE_PATH)
+        return str(e)
+
+
 def build(verbose: bool = False) -> str:
     """Compiles every csrc/*.hip to an object (in parallel, one hipcc per
     file) and links them into the shared library, and csrc/native.cpp into
-    the Python entry module beside it.  Always recompiles."""
+    the Python entry module beside it.  Always recompiles.  Without the entry
+    module the operators make their calls through ctypes, so a failure there
+    is a warning on stderr."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
     objs = [os.path.join(OBJ_DIR, os.path.basename(s)[:-4] + ".o") for s in srcs]
     jobs = max(1, min(len(srcs) + 1, os.cpu_count() or 1, 16))
-    native_tmp = NATIVE_PATH + ".tmp"
     with ThreadPoolExecutor(jobs) as ex:
-        native = ex.submit(_run, native_command(native_tmp), verbose)
+        native = ex.submit(build_native, verbose)
         list(ex.map(lambda so: _run([hipcc, *HIPCC_FLAGS, "-c", "-o", so[1], so[0]], verbose),
                     zip(srcs, objs)))
-        native.result()
-    os.replace(native_tmp, NATIVE_PATH)
+        failed = native.result()
     tmp = LIB_PATH + ".tmp"
     _run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp, *objs], verbose)
     os.replace(tmp, LIB_PATH)
+    if failed:
+        print(f"warning: {NATIVE_PATH} not built, calls go through ctypes: {failed}", file=sys.stderr)
     return LIB_PATH
 
 

@@ -275,3 +275,31 @@ def test_arguments_are_refused_without_the_library_too(monkeypatch, tmp_path, th
     monkeypatch.setattr(_lib, "require_gpu", lambda *t: torch.device("cpu"))
     with pytest.raises(_lib.KernelLibraryMissing if there == "nothing" else OSError):
         add_rmsnorm(x, None, p, 1e-6)
+
+
+def test_the_library_is_linked_without_the_cpp_entry(monkeypatch, tmp_path, capsys):
+    """The C++ entry is optional: without a host compiler or torch's headers the
+    build still ends with the library, says what failed, and leaves no older entry
+    module behind.  (Every compiler run is replaced by writing its output file.)"""
+    from spikeinfer_amd import build as b
+
+    made = []
+
+    def run(cmd, verbose):
+        out = cmd[cmd.index("-o") + 1]
+        if cmd[0].endswith("no-such-g++"):
+            raise FileNotFoundError(cmd[0])
+        made.append(out)
+        open(out, "w").close()
+
+    monkeypatch.setenv("CXX", "no-such-g++")
+    monkeypatch.setattr(b, "_run", run)
+    for name, file in (("OBJ_DIR", "obj"), ("LIB_PATH", "lib.so"), ("NATIVE_PATH", "_native.so")):
+        monkeypatch.setattr(b, name, str(tmp_path / file))
+    (tmp_path / "_native.so").write_text("older")
+    assert b.build() == str(tmp_path / "lib.so")
+    assert (tmp_path / "lib.so").exists() and not (tmp_path / "_native.so").exists()
+    assert "no-such-g++" in capsys.readouterr().err
+    monkeypatch.setenv("CXX", "g++")
+    b.build()
+    assert (tmp_path / "_native.so").exists()
