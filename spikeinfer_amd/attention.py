@@ -17,6 +17,7 @@ from __future__ import annotations
 from dataclasses import dataclass, field, replace
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 
 from .kernels.lif import lif_multistep, lif_pack_write_sites
@@ -74,6 +75,11 @@ class AttentionMetadata:
         return self._copies[key]
 
 
+def _carries_derivatives(t: torch.Tensor) -> bool:
+    """Whether derivatives to ``t`` flow on: reverse mode, or a forward-mode tangent."""
+    return (t.requires_grad and torch.is_grad_enabled()) or fwAD.unpack_dual(t).tangent is not None
+
+
 def _causal_offset_mask(query_len: int, total_len: int, device, dtype) -> torch.Tensor:
     """Additive mask letting query i (at position total_len - query_len + i)
     see positions <= its own (spikeinfer/attention.py:320-330)."""
@@ -95,7 +101,7 @@ def _prefill_packed(q_packed, first, k_cache, v_cache, meta, out, head_dim):
 def _prefill(q_dense, k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim):
     """The same from dense query spikes: one gather-unpack launch yields dense K
     and V, then SDPA with the offset causal mask.  For what the packed kernel
-    does not take (head_dim over 128) and for gradients to dense queries."""
+    does not take (head_dim over 128) and for derivatives to dense queries."""
     dtype, device = q_dense.dtype, q_dense.device
     for i in range(meta.num_prefills):
         start = meta.prefill_query_starts[i]
@@ -136,7 +142,7 @@ def paged_attention(
     out = torch.empty((T, n_tok, num_q_heads, head_dim), device=device, dtype=dtype)
     n_dec = meta.num_decode_tokens
     packed = bool(meta.num_prefills) and prefill_supported(head_dim, dtype) and \
-        not (q_spk.requires_grad and torch.is_grad_enabled())
+        not _carries_derivatives(q_spk)
     if packed:  # every token's query words at once: [T, n_tok, H_q, W]
         q_words = pack_spikes(q_spk[:, 0]).permute(0, 2, 1, 3)
     if n_dec:

@@ -1,0 +1,109 @@
+"""Which form of the prefill attention a call takes, and what it does with the
+forms of its arguments, on the CPU: the kernels' wrappers are replaced by plain
+torch, the packed kernel by a float64 evaluation of its words."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+import torch.autograd.forward_ad as fwAD
+from torch.nn.attention import SDPBackend, sdpa_kernel
+
+import spikeinfer_amd.attention as A
+from model_ref import gather_ref, lif_ref, pack_ref, unpack_ref
+from spikeinfer_amd.attention import AttentionMetadata, paged_attention
+from spikeinfer_amd.kernels.spike_attention import PREFILL_DTYPES
+
+T, HQ, HKV, D, BS = 2, 4, 2, 64, 16
+
+
+@pytest.fixture
+def packed_calls(monkeypatch):
+    """Plain torch in the kernels' place; the calls of the packed prefill kernel."""
+    calls = []
+
+    def prefill(q, k, v, chunks, out, head_dim, block_size):
+        # what the kernel's wrapper asks of them
+        assert out.stride(-1) == 1 and out.dtype in PREFILL_DTYPES
+        calls.append(chunks)
+        for q_row, out_row, n, ctx, table in chunks:
+            kd, vd = (gather_ref(c, table, ctx + n, head_dim, block_size, torch.float64) for c in (k, v))
+            qd = unpack_ref(q[:, q_row:q_row + n], head_dim, torch.float64).transpose(1, 2)
+            rep = qd.shape[1] // kd.shape[1]
+            s = qd @ kd.repeat_interleave(rep, 1).transpose(-1, -2) / math.sqrt(head_dim)
+            s = s.masked_fill(torch.arange(ctx + n) > ctx + torch.arange(n)[:, None], -math.inf)
+            out[:, out_row:out_row + n] = (torch.softmax(s, -1) @ vd.repeat_interleave(rep, 1)).transpose(1, 2)
+        return out
+
+    def sites(every, slots):
+        assert len({x.dtype for x, *_ in every}) == 1  # what the kernel's wrapper asks
+        for x, beta, th, out, scatter in every:
+            words = pack_ref(lif_ref(x, beta, th))
+            out.index_copy_(2, slots, words.transpose(1, 2)) if scatter else out.copy_(words)
+
+    def pack(x):
+        x.data_ptr()  # (raises for a tensor without storage, as the kernel's wrapper does)
+        return pack_ref(x)
+
+    monkeypatch.setattr(A, "pack_spikes", pack)
+    monkeypatch.setattr(A, "gather_kv_unpacked_pair",
+                        lambda k, v, *a: (gather_ref(k, *a), gather_ref(v, *a)))
+    monkeypatch.setattr(A, "paged_spike_attn_prefill", prefill)
+    monkeypatch.setattr(A, "lif_pack_write_sites", sites)
+    return calls
+
+
+def _spikes(n, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [(torch.rand((T, 1, h, n, D), generator=g) < 0.3).float() for h in (HQ, HKV, HKV)]
+
+
+def _meta(lens, ctx=None, tables=None):
+    n, starts = sum(lens), [sum(lens[:i]) for i in range(len(lens))]
+    tables = tables if tables is not None else [torch.arange(4 * i, 4 * i + 4).int() for i in range(len(lens))]
+    slots = torch.cat([4 * BS * i + torch.arange(m) for i, m in enumerate(lens)])
+    return AttentionMetadata(slot_mapping=slots, block_size=BS, prefill_query_starts=starts, prefill_query_lens=lens,
+                             prefill_context_lens=ctx or [0] * len(lens), prefill_block_tables=tables)
+
+
+def _caches():
+    return [torch.zeros((T, HKV, 12 * BS, 2), dtype=torch.int32) for _ in range(2)]
+
+
+def _attend(n):
+    """The step as a function of its queries."""
+    (_, k, v), caches, meta = _spikes(n), _caches(), _meta([n])
+    return lambda q: paged_attention(q, k, v, *caches, meta, HQ, HKV, D)
+
+
+def test_plain_queries_take_the_packed_kernel(packed_calls):
+    q, attend = _spikes(9)[0], _attend(9)
+    plain = attend(q)
+    with torch.no_grad():
+        off = attend(q.clone().requires_grad_())
+    assert len(packed_calls) == 2 and torch.equal(plain, off)
+    grad = attend(q.clone().requires_grad_())
+    assert len(packed_calls) == 2 and grad.requires_grad
+    torch.testing.assert_close(grad.detach(), plain, rtol=0, atol=1e-6)
+
+
+def test_derivatives_to_the_queries_flow_in_every_mode(packed_calls):
+    """Reverse and forward mode: neither may end in packed words.  (torch.func's
+    transforms wrap the k spikes too, which the packing refuses.)"""
+    q, attend = _spikes(9)[0], _attend(9)
+    d = torch.randn(q.shape, generator=torch.Generator().manual_seed(1))
+    leaf = q.clone().requires_grad_()
+    with sdpa_kernel(SDPBackend.MATH):  # (the only backend with a forward mode)
+        reverse = torch.autograd.grad(attend(leaf).square().sum(), leaf)[0]
+        with fwAD.dual_level():
+            out = fwAD.unpack_dual(attend(fwAD.make_dual(q, d)))
+            assert out.tangent is not None
+            forward = (2 * out.primal * out.tangent).sum()
+        with pytest.raises(RuntimeError, match="storage"):
+            torch.func.grad(lambda x: attend(x).sum())(q)
+    torch.testing.assert_close(forward, (reverse * d).sum(), rtol=1e-4, atol=1e-4)
+    assert not packed_calls
+    with fwAD.dual_level():  # a level without a tangent to the queries
+        attend(q)
+    assert len(packed_calls) == 1
