@@ -92,9 +92,9 @@ def _prefill_packed(q_packed, first, k_cache, v_cache, meta, out, head_dim):
     """Each prefill chunk attends to its sequence's whole cached prefix plus
     itself, straight from the packed words (spikeinfer/attention.py:161-178).
     Row ``i`` of ``q_packed [T, n, H_q, W]`` is batch row ``first + i``."""
-    chunks = [(start - first, start, q_len, ctx, table) for start, q_len, ctx, table in
-              zip(meta.prefill_query_starts, meta.prefill_query_lens, meta.prefill_context_lens,
-                  meta.prefill_block_tables)]
+    # (indexed: a list shorter than the others is an error)
+    chunks = [(meta.prefill_query_starts[i] - first, meta.prefill_query_starts[i], meta.prefill_query_lens[i],
+               meta.prefill_context_lens[i], meta.prefill_block_tables[i]) for i in range(meta.num_prefills)]
     paged_spike_attn_prefill(q_packed, k_cache, v_cache, chunks, out, head_dim, meta.block_size)
 
 

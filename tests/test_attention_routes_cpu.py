@@ -107,3 +107,19 @@ def test_derivatives_to_the_queries_flow_in_every_mode(packed_calls):
     with fwAD.dual_level():  # a level without a tangent to the queries
         attend(q)
     assert len(packed_calls) == 1
+
+
+def test_every_chunk_needs_its_entry_in_each_list(packed_calls):
+    """A list shorter than the chunks' lengths is an error, not rows left unwritten;
+    entries past them are not looked at."""
+    q, k, v = _spikes(12)
+    run = lambda meta: paged_attention(q, k, v, *_caches(), meta, HQ, HKV, D)
+    good = run(_meta([5, 7]))
+    for name in ("prefill_query_starts", "prefill_context_lens", "prefill_block_tables"):
+        meta = _meta([5, 7])
+        setattr(meta, name, getattr(meta, name)[:1])
+        with pytest.raises(IndexError):
+            run(meta)
+        meta = _meta([5, 7])
+        setattr(meta, name, getattr(meta, name) * 2)
+        assert torch.equal(run(meta), good)
