@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from .kernels.lif import lif_multistep, lif_pack_write_sites
 from .kernels.packing import pack_spikes, packed_width
-from .kernels.spike_attention import (gather_kv_unpacked_pair, paged_spike_attn_decode,
+from .kernels.spike_attention import (PREFILL_DTYPES, gather_kv_unpacked_pair, paged_spike_attn_decode,
                                       paged_spike_attn_prefill, prefill_supported)
 
 
@@ -88,14 +88,21 @@ def _causal_offset_mask(query_len: int, total_len: int, device, dtype) -> torch.
     return torch.triu(mask, diagonal=ctx + 1)
 
 
-def _prefill_packed(q_packed, first, k_cache, v_cache, meta, out, head_dim):
+def _prefill_packed(q_packed, first, k_cache, v_cache, meta, out, head_dim, dtype):
     """Each prefill chunk attends to its sequence's whole cached prefix plus
     itself, straight from the packed words (spikeinfer/attention.py:161-178).
-    Row ``i`` of ``q_packed [T, n, H_q, W]`` is batch row ``first + i``."""
+    Row ``i`` of ``q_packed [T, n, H_q, W]`` is batch row ``first + i``; values
+    are rounded to ``dtype`` on the way to an ``out`` the kernel does not write."""
     # (indexed: a list shorter than the others is an error)
     chunks = [(meta.prefill_query_starts[i] - first, meta.prefill_query_starts[i], meta.prefill_query_lens[i],
                meta.prefill_context_lens[i], meta.prefill_block_tables[i]) for i in range(meta.num_prefills)]
-    paged_spike_attn_prefill(q_packed, k_cache, v_cache, chunks, out, head_dim, meta.block_size)
+    dst = out
+    if out.dtype not in PREFILL_DTYPES or out.stride(-1) != 1:  # (the kernel's outputs)
+        dst = torch.empty(out.shape, dtype=dtype, device=out.device)
+    paged_spike_attn_prefill(q_packed, k_cache, v_cache, chunks, dst, head_dim, meta.block_size)
+    if dst is not out:
+        for _, start, q_len, _, _ in chunks:
+            out[:, start:start + q_len] = dst[:, start:start + q_len]
 
 
 def _prefill(q_dense, k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim):
@@ -153,7 +160,7 @@ def paged_attention(
             num_kv_heads=num_kv_heads, out=out[:, :n_dec],
         )
     if packed:
-        _prefill_packed(q_words, 0, k_cache, v_cache, meta, out, head_dim)
+        _prefill_packed(q_words, 0, k_cache, v_cache, meta, out, head_dim, dtype)
     elif meta.num_prefills:
         _prefill(q_spk[:, 0], k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim)
     return out.view(T, 1, n_tok, num_q_heads * head_dim)
@@ -218,7 +225,7 @@ def paged_attention_fused(
             num_kv_heads=num_kv_heads, out=out[:, :n_dec],
         )
     if packed:
-        _prefill_packed(q_words, n_dec, k_cache, v_cache, meta, out, head_dim)
+        _prefill_packed(q_words, n_dec, k_cache, v_cache, meta, out, head_dim, dtype)
     elif meta.num_prefills:
         # Prefill queries need dense spikes for SDPA; the LIF is per token, so
         # running it on the prefill tokens alone gives the same spikes.

@@ -12,7 +12,7 @@ from torch.nn.attention import SDPBackend, sdpa_kernel
 
 import spikeinfer_amd.attention as A
 from model_ref import gather_ref, lif_ref, pack_ref, unpack_ref
-from spikeinfer_amd.attention import AttentionMetadata, paged_attention
+from spikeinfer_amd.attention import AttentionMetadata, paged_attention, paged_attention_fused
 from spikeinfer_amd.kernels.spike_attention import PREFILL_DTYPES
 
 T, HQ, HKV, D, BS = 2, 4, 2, 64, 16
@@ -123,3 +123,25 @@ def test_every_chunk_needs_its_entry_in_each_list(packed_calls):
         meta = _meta([5, 7])
         setattr(meta, name, getattr(meta, name) * 2)
         assert torch.equal(run(meta), good)
+
+
+def _fused(n, out=None, q_dtype=torch.float32, **over):
+    g = torch.Generator().manual_seed(n)
+    cur = [torch.randn((T, n, h, D), generator=g) for h in (HQ, HKV, HKV)]
+    cur[0] = cur[0].bfloat16().to(q_dtype)
+    lif = [(torch.full((D,), 0.9), torch.full((D,), 1.0))] * 3
+    return paged_attention_fused(*cur, *lif, *_caches(), _meta([5, n - 5]), HQ, HKV, D, out=out)
+
+
+def test_fused_outputs_of_any_type_and_layout(packed_calls):
+    """The kernel writes floats with contiguous channels; other `out` tensors
+    receive the chunks' rows too, and nothing else of them is touched."""
+    n = 12
+    want = _fused(n)
+    for dtype, step in ((torch.float64, 1), (torch.float32, 2), (torch.bfloat16, 2)):
+        big = torch.full((T, n + 2, HQ, step * D), -7.0, dtype=dtype)
+        out = big[:, :n, :, ::step]
+        got = _fused(n, out)
+        assert got.dtype == dtype and got.data_ptr() == big.data_ptr()
+        assert torch.equal(got, want.to(dtype))
+        assert (big[:, n:] == -7).all() and (step == 1 or (big[:, :, :, 1::step] == -7).all())
