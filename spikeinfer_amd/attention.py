@@ -216,7 +216,11 @@ def paged_attention_fused(
     if packed:
         q_words = torch.empty((T, n_tok - n_dec, num_q_heads, packed_width(head_dim)), dtype=torch.int32,
                               device=device)
-        sites.append((q_cur[:, n_dec:], lif_q[0], lif_q[1], q_words, False))
+        q_site = (q_cur[:, n_dec:], lif_q[0], lif_q[1], q_words, False)
+        if dtype == k_cur.dtype:
+            sites.append(q_site)
+        else:  # (the sites of a launch share one type)
+            lif_pack_write_sites([q_site])
     lif_pack_write_sites(sites, meta.slot_mapping)
     if n_dec:
         paged_spike_attn_decode(

@@ -145,3 +145,10 @@ def test_fused_outputs_of_any_type_and_layout(packed_calls):
         assert got.dtype == dtype and got.data_ptr() == big.data_ptr()
         assert torch.equal(got, want.to(dtype))
         assert (big[:, n:] == -7).all() and (step == 1 or (big[:, :, :, 1::step] == -7).all())
+
+
+def test_fused_query_currents_of_their_own_type(packed_calls):
+    """Query currents in another float type than k and v (one launch takes one type)."""
+    want = _fused(12)
+    got = _fused(12, q_dtype=torch.bfloat16)
+    assert got.dtype == torch.bfloat16 and torch.equal(got, want.bfloat16())
