@@ -36,7 +36,7 @@ def packed_calls(monkeypatch):
             out[:, out_row:out_row + n] = (torch.softmax(s, -1) @ vd.repeat_interleave(rep, 1)).transpose(1, 2)
         return out
 
-    def sites(every, slots):
+    def sites(every, slots=None):
         assert len({x.dtype for x, *_ in every}) == 1  # what the kernel's wrapper asks
         for x, beta, th, out, scatter in every:
             words = pack_ref(lif_ref(x, beta, th))
