@@ -20,7 +20,7 @@ import torch
 import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 
-from .kernels.lif import lif_multistep, lif_pack_write_sites
+from .kernels.lif import lif_pack_write_sites
 from .kernels.packing import pack_spikes, packed_width
 from .kernels.spike_attention import (PREFILL_DTYPES, gather_kv_unpacked_pair, paged_spike_attn_decode,
                                       paged_spike_attn_prefill, prefill_supported)
@@ -191,7 +191,8 @@ def paged_attention_fused(
 
     Args:
         q_cur, k_cur, v_cur: ``[T, n_tok, H, D]`` currents (any strides, e.g.
-            ``proj_out.view(T, n_tok, H, D)`` of the projection + RoPE output).
+            ``proj_out.view(T, n_tok, H, D)`` of the projection + RoPE output);
+            fp32, fp16 or bf16, head_dim at most 128 (the LIF-pack launch's range).
         lif_q, lif_k, lif_v: ``(beta, threshold)`` of each site, ``[D]`` each.
         out: optional preallocated ``[T, n_tok, H_q, D]`` in the currents' dtype.
         q_packed: optional preallocated ``int32 [T, n_dec, H_q, W]`` buffer.
@@ -212,8 +213,7 @@ def paged_attention_fused(
             q_packed = torch.empty((T, n_dec, num_q_heads, packed_width(head_dim)),
                                    dtype=torch.int32, device=device)
         sites.append((q_cur[:, :n_dec], lif_q[0], lif_q[1], q_packed, False))
-    packed = bool(meta.num_prefills) and prefill_supported(head_dim, dtype)
-    if packed:
+    if meta.num_prefills:
         q_words = torch.empty((T, n_tok - n_dec, num_q_heads, packed_width(head_dim)), dtype=torch.int32,
                               device=device)
         q_site = (q_cur[:, n_dec:], lif_q[0], lif_q[1], q_words, False)
@@ -228,13 +228,6 @@ def paged_attention_fused(
             head_dim=head_dim, block_size=meta.block_size, num_q_heads=num_q_heads,
             num_kv_heads=num_kv_heads, out=out[:, :n_dec],
         )
-    if packed:
+    if meta.num_prefills:
         _prefill_packed(q_words, n_dec, k_cache, v_cache, meta, out, head_dim, dtype)
-    elif meta.num_prefills:
-        # Prefill queries need dense spikes for SDPA; the LIF is per token, so
-        # running it on the prefill tokens alone gives the same spikes.
-        q_pre = lif_multistep(q_cur[:, n_dec:], lif_q[0], lif_q[1])  # [T, n_pre, H_q, D]
-        q_dense = torch.zeros((T, num_q_heads, n_tok, head_dim), device=device, dtype=dtype)
-        q_dense[:, :, n_dec:] = q_pre.permute(0, 2, 1, 3)
-        _prefill(q_dense, k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim)
     return out.view(T, 1, n_tok, num_q_heads * head_dim)

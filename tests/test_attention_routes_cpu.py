@@ -152,3 +152,33 @@ def test_fused_query_currents_of_their_own_type(packed_calls):
     want = _fused(12)
     got = _fused(12, q_dtype=torch.bfloat16)
     assert got.dtype == torch.bfloat16 and torch.equal(got, want.bfloat16())
+
+
+@pytest.mark.parametrize("lens,ctx", [([20, 20, 20], [0, 0, 0]), ([20, 33, 1], [0, 0, 0]),
+                                      ([7, 20, 20], [40, 0, 0]), ([9, 5], [33, 20])])
+def test_dense_prefill_of_wide_heads(monkeypatch, lens, ctx):
+    """SpikingDecoder's dense form, which heads of more than 128 channels take: fresh
+    chunks of one length in one batched call, ragged ones, and cached prefixes."""
+    import spikeinfer_amd.model as M
+
+    D, n = 256, sum(lens)
+    g = torch.Generator().manual_seed(n)
+    monkeypatch.setattr(M, "gather_kv_unpacked_pair", lambda k, v, *a: (gather_ref(k, *a), gather_ref(v, *a)))
+    caches = [pack_ref((torch.rand((T, HKV, 12 * BS, D), generator=g) < 0.3).float()) for _ in range(2)]
+    dense = [(torch.rand((T, h, n, D), generator=g) < 0.3).float() for h in (HQ, HKV, HKV)]
+    meta = _meta(lens, ctx)
+    for i, (start, m, c) in enumerate(zip(meta.prefill_query_starts, lens, ctx)):  # the chunk's own k and v
+        for cache, d in zip(caches, dense[1:]):
+            cache[:, :, 4 * BS * i + c:4 * BS * i + c + m] = pack_ref(d[:, :, start:start + m])
+    model = M.SpikingDecoder.__new__(M.SpikingDecoder)
+    model.T, model.D, model.Hq, model.Hkv, model.dtype = T, D, HQ, HKV, torch.float32
+    attn = torch.full((T, n, HQ, D), float("nan"))
+    model._prefill_attention(dense, *caches, meta, attn)
+    for i, (start, m, c) in enumerate(zip(meta.prefill_query_starts, lens, ctx)):
+        k, v = (gather_ref(x, meta.prefill_block_tables[i], c + m, D, BS, torch.float64) for x in caches)
+        q = dense[0][:, :, start:start + m].double()
+        s = q @ k.repeat_interleave(HQ // HKV, 1).transpose(-1, -2) / math.sqrt(D)
+        s = s.masked_fill(torch.arange(c + m) > c + torch.arange(m)[:, None], -math.inf)
+        want = (torch.softmax(s, -1) @ v.repeat_interleave(HQ // HKV, 1)).transpose(1, 2)
+        # (values in [0, 1], at most 49 fp32 terms: 49 * 2**-24)
+        torch.testing.assert_close(attn[:, start:start + m].double(), want, rtol=0, atol=3e-6)

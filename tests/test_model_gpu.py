@@ -567,7 +567,7 @@ def test_incremental_decode_matches_whole_prefill(gpu):
     single-token decode steps (reference: tests/test_kv_cache.py:87-126,
     incremental decode vs full-prefix recompute).  The decode steps run the
     decode kernels (fused attention, small-M GEMMs, fused MLP), the chunk the
-    prefill path (library GEMMs, SDPA on the dense spikes), so the two round
+    prefill path (library GEMMs, attention on packed words), so the two round
     differently and a spike on its threshold may flip: the last token's hidden
     state and the caches are held to the model tests' bounds, and the next
     token must agree."""
