@@ -21,8 +21,9 @@
 //   * A score is an integer in 0..head_dim, so its weight exp(score * scale) is a
 //     table entry at byte 4 * score: (hi, lo) halves of an f16 pair with hi + lo
 //     the weight to 2^-23 (the table spans e^sqrt(head_dim) <= 2^17 below 2^15, so
-//     both halves are normal or lose nothing that counts).  Lookups do not
-//     conflict: different entries lie in different banks, equal ones broadcast.
+//     both halves are normal or lose nothing that counts).  Equal entries broadcast
+//     and different ones lie in different banks, save scores 64 apart (0 and 64
+//     at head_dim 64; at 128, s and s + 64, far apart for words of one density).
 //     No running maximum, no rescaling: any fixed offset cancels in a / l.
 //   * Values: O^T[channel, row] += V^T P^T with v_mfma_f32_32x32x16_f16 over
 //     (key, hi/lo) pairs.  The score layout (lane l: row l % 32, keys 4 * (l / 32) +
@@ -32,8 +33,16 @@
 //     it is built once per key tile and shared by the QT row tiles.
 //   * Denominators: v_dot2_f32_f16 of the pair with (1, 1), 16 weights to a
 //     partial sum and the partial sums in fp32 (one long dot2 chain per row lost
-//     1e-6 at 4,000 keys).  Error against float64, fp32 output: 4.1e-7 at 4,000
-//     keys, 4.6e-7 at 16,000; fp32 SDPA 7.9e-7 and 1.3e-5.
+//     1e-6 at 4,000 keys).
+//   * fp32 outputs take the hi and the lo products to accumulators of their own, two
+//     keys a register (v_perm), the same number of instructions of the matrix cores.
+//     Sums of 11-bit halves are exact in fp32 until they pass 2^24 of the smallest
+//     one's units, so the sums lose next to nothing; they are added, and divided, in
+//     fp64 and rounded once.  Error against float64 in the 2-norm, head_dim 32 to
+//     128, 2 to 12,000 keys, a fifth or half of the bits set: 1.6e-8 to 4.1e-8;
+//     one accumulator with rounded sums 3.1e-8 to 7e-8 up to 64 keys and up to
+//     1.6e-6 beyond; fp32 SDPA 2.7e-8 to 1.1e-7 and up to 1e-5.  The prompt below
+//     172 us against 143 with one accumulator, whose bits 16-bit outputs do not show.
 // What bounds it: issue.  A 32 x 32 tile at head_dim 64 takes 288 cycles of matrix
 // core (two f16 products a weight keep it at 32-bit precision) and about 330 of
 // VALU, and the two overlap little: 720 measured (a 4,096-token prompt, 14 / 2
@@ -130,16 +139,19 @@ __device__ __forceinline__ v8i fp4_bits(uint32_t w) {
 }
 
 // QT row tiles of 32 rows a workgroup; NC = channel tiles of 32 (ceil(D / 32)).
-template <int QT, int NC>
+// F32: the outputs are fp32.
+template <int QT, int NC, bool F32>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(
     Params p) {
   constexpr int NK = (NC + 1) / 2;         // 64-channel score steps
   constexpr int kUnits = QT * NC;          // 32 x 32 output tiles a workgroup
-  constexpr int kRounds = (kUnits + kWaves - 1) / kWaves;
+  constexpr int kParts = F32 ? 2 : 1;      // accumulators of a tile: the hi and the lo products apart
+  constexpr int kTiles = kWaves / kParts;  // output tiles a round of the final sums
+  constexpr int kRounds = (kUnits + kTiles - 1) / kTiles;
   struct Smem {
     uint32_t tab[kTab + 3];  // first: a score's accumulator is its entry's LDS address
-    float lsum[QT][kWaves][64];
-    float red[kUnits < kWaves ? kUnits : kWaves][kWaves][16][64];
+    float lsum[QT][kParts][kWaves][64];
+    float red[kUnits * kParts < kWaves ? kUnits * kParts : kWaves][kWaves][16][64];
   };
   __shared__ Smem sm;
   auto &tab = sm.tab;
@@ -215,13 +227,14 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
   };
   auto keep = [&](uint32_t x, int s, bool ok) { return ok && 2 * s + half < p.W ? x : 0u; };
 
-  v16f acc[QT][NC];
-  float l[QT];
+  v16f acc[QT][NC * kParts];
+  float l[QT][kParts];
 #pragma unroll
   for (int i = 0; i < QT; ++i) {
-    l[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[i][c] = v16f{};
+    for (int p2 = 0; p2 < kParts; ++p2) l[i][p2] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC * kParts; ++c) acc[i][c] = v16f{};
   }
   __syncthreads();
 
@@ -247,15 +260,21 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
     }
     load(kt + kWaves, pnext, kw, vw, ok);
     pnext = block_of(kt + 2 * kWaves);
-    v8h vop[NC][4];
+    v8h vop[NC][4 / kParts];
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int g = 0; g < 4 / kParts; ++g) {
         v4u x;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          x[i] = static_cast<uint32_t>(static_cast<int>(vt[c] << (31 - 8 * g - i)) >> 31) & 0x3c003c00u;
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (F32) {  // two keys a register
+            const uint32_t b = vt[c] >> (16 * g + 8 * (i >> 1) + 2 * (i & 1));
+            x[i] = ((b & 1u) | ((b & 2u) << 15)) * 0x3c00u;
+          } else {
+            x[i] = static_cast<uint32_t>(static_cast<int>(vt[c] << (31 - 8 * g - i)) >> 31) & 0x3c003c00u;
+          }
+        }
         vop[c][g] = __builtin_bit_cast(v8h, x);
       }
     auto scores = [&](int i) {
@@ -273,23 +292,54 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
       }
     };
     auto products = [&](int i, const uint32_t (&w)[16], auto masked) {
+      auto weight = [&](int n) {  // the n-th of the lane's sixteen
+        if constexpr (decltype(masked)::value)
+          return kt * kKeys + 8 * (n >> 2) + 4 * half + (n & 3) <= lim[i] ? w[n] : 0u;
+        else return w[n];
+      };
       float d[4] = {0.f, 0.f, 0.f, 0.f};  // (a chain of dot2 on one register waits for itself)
+      if constexpr (F32) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        v4u x;
+        for (int g = 0; g < 2; ++g) {
+          v4u x[2];  // hi and lo halves, two keys a register
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          uint32_t y = w[4 * g + e];
-          if constexpr (decltype(masked)::value) y = kt * kKeys + 8 * g + 4 * half + e <= lim[i] ? y : 0u;
-          d[e] = __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, y), v2h{1, 1}, d[e], false);
-          x[e] = y;
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t y0 = weight(8 * g + 2 * e), y1 = weight(8 * g + 2 * e + 1);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const uint32_t y = __builtin_amdgcn_perm(y1, y0, q ? 0x07060302u : 0x05040100u);
+              float &dq = d[2 * (e & 1) + q];
+              dq = __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, y), v2h{1, 1}, dq, false);
+              x[q][e] = y;
+            }
+          }
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              v16f &a = acc[i][2 * c + q];
+              a = __builtin_amdgcn_mfma_f32_32x32x16_f16(vop[c][g], __builtin_bit_cast(v8h, x[q]), a, 0, 0, 0);
+            }
         }
-        const v8h pw = __builtin_bit_cast(v8h, x);
+        l[i][0] += d[0] + d[2];
+        l[i][kParts - 1] += d[1] + d[3];
+      } else {
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-          acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vop[c][g], pw, acc[i][c], 0, 0, 0);
+        for (int g = 0; g < 4; ++g) {
+          v4u x;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t y = weight(4 * g + e);
+            d[e] = __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, y), v2h{1, 1}, d[e], false);
+            x[e] = y;
+          }
+          const v8h pw = __builtin_bit_cast(v8h, x);
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+            acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vop[c][g], pw, acc[i][c], 0, 0, 0);
+        }
+        l[i][0] += (d[0] + d[1]) + (d[2] + d[3]);
       }
-      l[i] += (d[0] + d[1]) + (d[2] + d[3]);
     };
     if (nq == QT && kt * kKeys + kKeys - 1 <= lo[0]) {
       // The next row tile's scores are computed and looked up under this one's
@@ -315,47 +365,59 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
     }
   }
 
-  // Sums of the four waves, in wave order: each round the waves put four of the
-  // output tiles (row tile i, channel tile c) into LDS and wave w finishes the
-  // w-th of them.
+  // Sums of the four waves, in wave order: each round the waves put kTiles of the
+  // output tiles (row tile i, channel tile c) into LDS and each finishes one of them,
+  // or, of an fp32 tile in two parts, one half.
 #pragma unroll
-  for (int i = 0; i < QT; ++i) lsum[i][wave][lane] = l[i];
+  for (int i = 0; i < QT; ++i)
+#pragma unroll
+    for (int q = 0; q < kParts; ++q) lsum[i][q][wave][lane] = l[i][q];
 #pragma unroll
   for (int rd = 0; rd < kRounds; ++rd) {
     if (rd) __syncthreads();
 #pragma unroll
     for (int u = 0; u < kWaves; ++u) {
       constexpr int kU = kUnits;
-      const int x = rd * kWaves + u;
+      const int x = rd * kTiles + u / kParts;
       if (x < kU) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) red[u][wave][j][lane] = acc[x / NC][x % NC][j];
+        for (int j = 0; j < 16; ++j) red[u][wave][j][lane] = acc[x / NC][x % NC * kParts + u % kParts][j];
       }
     }
     __syncthreads();
-    const int x = rd * kWaves + wave;
+    const int x = rd * kTiles + wave / kParts;
     const int i = x / NC, c = x - i * NC;
     const int r = r0 + 32 * i + col;
     if (x >= kUnits || r >= rows) continue;
-    float den = 0.f;
+    const int slot = wave / kParts * kParts;        // the tile's place in red
+    const int g0 = F32 ? wave % kParts * 2 : 0;      // first of the wave's 4-channel groups
+    constexpr int kGroups = F32 ? 2 : 4;
+    // fp32 outputs: the parts' sums and the quotient in fp64, rounded once.
+    typedef std::conditional_t<F32, double, float> Sum;
+    Sum den = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) den += lsum[i][w][col] + lsum[i][w][col + 32];
-    const float inv = 1.f / den;
+    for (int q = 0; q < kParts; ++q)
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w)
+        den += static_cast<Sum>(lsum[i][q][w][col]) + static_cast<Sum>(lsum[i][q][w][col + 32]);
+    const Sum inv = Sum(1) / den;
     const int tok = token_of(r), h = r - tok * p.nrep;
     const int64_t row = t * p.os0 + (start + tok) * p.os1 + (kvh * p.nrep + h) * p.os2;
     auto value = [&](int j) {
-      float a = 0.f;
+      Sum a = 0;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) a += red[wave][w][j][lane];
-      return a * inv;
+      for (int q = 0; q < kParts; ++q)
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) a += red[slot + q][w][j][lane];
+      return static_cast<float>(a * inv);
     };
     if (p.out_vec) {  // D % 4 == 0: four channels lie in or out together
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int ch = 32 * c + 8 * g + 4 * half;
+      for (int k = 0; k < kGroups; ++k) {
+        const int g = g0 + k, ch = 32 * c + 8 * g + 4 * half;
         const float o[4] = {value(4 * g), value(4 * g + 1), value(4 * g + 2), value(4 * g + 3)};
         if (ch >= p.D) continue;
-        if (p.out_dtype == SPK_F32) {
+        if constexpr (F32) {
           *reinterpret_cast<v4f *>(static_cast<float *>(p.out) + row + ch) = v4f{o[0], o[1], o[2], o[3]};
           continue;
         }
@@ -376,7 +438,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
       }
     } else {
 #pragma unroll 1
-      for (int j = 0; j < 16; ++j) {
+      for (int j = 4 * g0; j < 4 * (g0 + kGroups); ++j) {
         const int ch = 32 * c + 8 * (j >> 2) + 4 * half + (j & 3);
         if (ch < p.D) store_f32_as(p.out, row + ch, p.out_dtype, value(j));
       }
@@ -405,13 +467,20 @@ static void build_table(float scale, int D, uint32_t *tab) {
   std::memcpy(tab, last, sizeof(uint32_t) * (D + 1));
 }
 
-template <int QT>
+// Row tiles a workgroup takes of the `qt` asked for: as many as its sums leave
+// registers for (fp32 outputs have two accumulators a tile).
+constexpr int row_tiles(int qt, int NC, bool f32) {
+  const int most = NC > 3 ? 1 : (NC > 2 ? (f32 ? 1 : 2) : (f32 ? 2 : 4));
+  return qt < most ? qt : most;
+}
+
+template <int QT, bool F32>
 static void launch(const Params &p, unsigned grid, hipStream_t s) {
   switch ((p.D + 31) / 32) {
-    case 1: prefill_attn_kernel<QT, 1><<<grid, kWaves * 64, 0, s>>>(p); break;
-    case 2: prefill_attn_kernel<QT, 2><<<grid, kWaves * 64, 0, s>>>(p); break;
-    case 3: prefill_attn_kernel<QT < 2 ? QT : 2, 3><<<grid, kWaves * 64, 0, s>>>(p); break;
-    default: prefill_attn_kernel<1, 4><<<grid, kWaves * 64, 0, s>>>(p); break;
+    case 1: prefill_attn_kernel<row_tiles(QT, 1, F32), 1, F32><<<grid, kWaves * 64, 0, s>>>(p); break;
+    case 2: prefill_attn_kernel<row_tiles(QT, 2, F32), 2, F32><<<grid, kWaves * 64, 0, s>>>(p); break;
+    case 3: prefill_attn_kernel<row_tiles(QT, 3, F32), 3, F32><<<grid, kWaves * 64, 0, s>>>(p); break;
+    default: prefill_attn_kernel<row_tiles(QT, 4, F32), 4, F32><<<grid, kWaves * 64, 0, s>>>(p); break;
   }
 }
 
@@ -473,7 +542,8 @@ extern "C" int spk_prefill_attn(const int32_t *q, const int64_t q_strides[3], co
   // not depend on it.
   const int64_t tiles = (total + 31) / 32 * p.units;
   const int qt = tiles >= 4 * 512 ? 4 : (tiles >= 2 * 512 ? 2 : 1);
-  const int qt_used = head_dim > 96 ? 1 : (head_dim > 64 && qt > 2 ? 2 : qt);
+  const bool f32 = out_dtype == SPK_F32;
+  const int qt_used = prefill::row_tiles(qt, p.W, f32);
   hipStream_t s = static_cast<hipStream_t>(stream);
   for (int i = 0; i < nchunks;) {
     int64_t grid = 0;
@@ -496,9 +566,16 @@ extern "C" int spk_prefill_attn(const int32_t *q, const int64_t q_strides[3], co
     }
     if (!p.nchunks) break;
     const unsigned g = static_cast<unsigned>(grid * p.units);
-    if (qt == 4) prefill::launch<4>(p, g, s);
-    else if (qt == 2) prefill::launch<2>(p, g, s);
-    else prefill::launch<1>(p, g, s);
+    if (f32) {
+      if (qt >= 2) prefill::launch<2, true>(p, g, s);
+      else prefill::launch<1, true>(p, g, s);
+    } else if (qt == 4) {
+      prefill::launch<4, false>(p, g, s);
+    } else if (qt == 2) {
+      prefill::launch<2, false>(p, g, s);
+    } else {
+      prefill::launch<1, false>(p, g, s);
+    }
     const int rc = check_launch("prefill_attn");
     if (rc) return rc;
   }

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from model_ref import gather_ref, pack_ref
-from spikeinfer_amd import _lib
+from spikeinfer_amd import _lib, attention
 from spikeinfer_amd.attention import AttentionMetadata, paged_attention
 from spikeinfer_amd.kernels.spike_attention import paged_spike_attn_prefill
 
@@ -85,6 +85,36 @@ def test_dense_and_silent_words(gpu):
             paged_spike_attn_prefill(q, k, v, [(0, 0, 70, 30, tables[0])], out, D, 16)
             kd, vd = (gather_ref(x, tables[0], 100, D, 16, torch.float64) for x in (k, v))
             assert (out.double() - _want(q, kd, vd, 30, D)).abs().max().item() <= TOL[torch.float32]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("density", [0.2, 0.5])
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 14, 2), (32, 8, 8), (128, 8, 2), (96, 6, 2), (45, 6, 2)])
+def test_fp32_outputs_keep_32_bits(gpu, D, Hq, Hkv, density):
+    """fp32 outputs against float64 by the keys a row sees, and against the fp32
+    composition (unpack-gather + SDPA).  The quotient is rounded once (at most 2**-24
+    of the value, 3.4e-8 in the 2-norm); a weight is exact to 2**-23, and what its
+    error leaves in a quotient of sums made of the same weights is below a third of
+    that; sums of the weights' high halves are exact up to 2**24 of the smallest one's
+    units.  So 4.5e-8 in the 2-norm, for short rows and long.  A row of one key is
+    exact."""
+    bits = lambda w: ((w.long()[..., None] >> torch.arange(32, device=gpu)) & 1).flatten(-2)[..., :D]
+    for n, ctx, edges in ((300, 0, (1, 2, 4, 8, 16, 32, 64, 128, 300)), (64, 3900, (3964,)), (32, 12000, (12032,))):
+        q, k, v, tables, _ = _case(2, Hq, Hkv, D, 16, [(n, ctx)], n + D, gpu, density, density)
+        out, sdpa = (torch.empty((2, n, Hq, D), device=gpu) for _ in range(2))
+        paged_spike_attn_prefill(q, k, v, [(0, 0, n, ctx, tables[0])], out, D, 16)
+        meta = AttentionMetadata(slot_mapping=torch.arange(n, device=gpu), block_size=16, prefill_query_starts=[0],
+                                 prefill_query_lens=[n], prefill_context_lens=[ctx], prefill_block_tables=tables)
+        attention._prefill(bits(q).float().transpose(1, 2), k, v, meta, sdpa, Hq, Hkv, D)
+        kd, vd = (gather_ref(x, tables[0], n + ctx, D, 16, torch.float64) for x in (k, v))
+        want = _want(q, kd, vd, ctx, D)
+        at = 0
+        for edge in edges:
+            rows = slice(at, edge - ctx)
+            rel = [((o[:, rows].double() - want[:, rows]).norm() / want[:, rows].norm()).item() for o in (out, sdpa)]
+            print(f"D={D} density={density} up to {edge} keys: {rel[0]:.2e}, sdpa {rel[1]:.2e}", flush=True)
+            assert rel[0] <= (0.0 if edge == 1 else 4.5e-8), (edge, rel)
+            at = edge - ctx
 
 
 @pytest.mark.gpu
