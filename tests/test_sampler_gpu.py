@@ -22,6 +22,10 @@ pytestmark = pytest.mark.gpu
 def _run(gpu, logits, params, histories, uniforms, dtype=torch.float32, sliced=False):
     n, V = logits.shape
     lg = torch.from_numpy(logits).to(gpu, dtype)
+    if sliced is not False and V % 8:  # the sliced stages take rows that start at 16 bytes
+        rows16 = torch.full((n, -(-V // 8) * 8), float("inf"), dtype=dtype, device=gpu)
+        rows16[:, :V] = lg
+        lg = rows16[:, :V]
     f = lambda k, dflt: torch.tensor([p.get(k, dflt) for p in params], dtype=torch.float32, device=gpu)
     cap = max(1, max(len(h) for h in histories))
     hist = torch.zeros((n, cap), dtype=torch.int64, device=gpu)
@@ -34,7 +38,8 @@ def _run(gpu, logits, params, histories, uniforms, dtype=torch.float32, sliced=F
         torch.tensor([p.get("top_k", -1) for p in params], dtype=torch.int32, device=gpu),
         f("top_p", 1.0), f("min_p", 0.0), f("rep", 1.0), f("presence", 0.0), f("frequency", 0.0),
         hist, hlen, torch.tensor(uniforms, dtype=torch.float32, device=gpu),
-        workspace=torch.empty(sample_workspace_bytes(n), dtype=torch.uint8, device=gpu) if sliced else None)
+        workspace=sliced if isinstance(sliced, torch.Tensor) else
+        torch.empty(sample_workspace_bytes(n), dtype=torch.uint8, device=gpu) if sliced else None)
     return out.cpu().tolist(), lg.float().cpu().numpy()
 
 
@@ -126,7 +131,7 @@ def test_sampler_sliced_candidates_give_the_same_tokens(gpu, case, dtype):
 SLICED_EDGE_CASES = [
     (12000, 3.0, dict(temperature=1.0, top_k=256)),               # fewer threads with elements than k: over 1,024 elements
     (5000, 3.0, dict(temperature=1.0, top_k=200, top_p=0.99)),    # the same, every element a candidate
-    (4099, 3.0, dict(temperature=0.9, top_k=40, rep=1.2)),        # a last slice of three elements
+    (4099, 3.0, dict(temperature=0.9, top_k=40, rep=1.2)),        # a sixth slice of 259, two without elements
     (65536, 3.0, dict(temperature=1.0, top_k=256)),
     (65537, 3.0, dict(temperature=1.0, top_k=50)),
     (163840, 3.0, dict(temperature=0.6, top_k=50, top_p=0.9)),
@@ -153,6 +158,40 @@ def test_sampler_sliced_bound_edges(gpu, case, dtype):
     plain, _ = _run(gpu, logits, [p] * rows, histories, us, dtype)
     sliced, _ = _run(gpu, logits, [p] * rows, histories, us, dtype, sliced=True)
     assert sliced == plain
+
+
+def _list_counts(ws, rows):
+    """[rows, 8] entries of each slice's list in a workspace (behind the values and
+    indices of 256 a slice), -1 where the slice leaves its row to the row kernel."""
+    return ws[rows * 8 * 256 * 8:].view(torch.int32)[:rows * 8].view(rows, 8).cpu().numpy()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", range(len(SLICED_EDGE_CASES)))
+def test_sampler_slices_list_their_largest(gpu, case, dtype):
+    """Which slices of such rows list their min(k, length) largest, and which must
+    leave it to the row kernel: those with over 1,024 candidates at the bound, the
+    k-th largest of the threads' largest.  (A bound that gathers too much gives the
+    right tokens as well, by way of the row kernel.)"""
+    V, scale, p = SLICED_EDGE_CASES[case]
+    rng = np.random.default_rng(300 + case)
+    rows, k = 12, p["top_k"]
+    logits = (rng.standard_normal((rows, V)) * scale).astype(np.float32)
+    logits[4, 100:] = -np.inf
+    logits[5, : V // 2] = 0.0
+    ws = torch.full((sample_workspace_bytes(rows),), 0x7f, dtype=torch.uint8, device=gpu)
+    _run(gpu, logits, [p] * rows, [[]] * rows, [0.5] * rows, dtype, sliced=ws)
+    counts = _list_counts(ws, rows)
+    length = -(-(-(-V // 8)) // 256) * 256
+    n = np.clip(V - np.arange(8) * length, 0, length)
+    listed = np.minimum(k, n)
+    plain = [r for r in range(rows) if r not in (4, 5)]
+    assert (counts[plain] == listed).all(), counts[plain]
+    # row 4: a run of 100 finite logits, 16 bytes a thread; with fewer such threads than k
+    # the bound is -infinity there too
+    finite = np.where(np.arange(8) == 0, -(-100 // (16 // dtype.itemsize)), 0)
+    assert (counts[4] == np.where((finite < k) & (n > 1024), -1, listed)).all(), counts[4]
+    assert (counts[5][:3] == (-1 if n[0] > 1024 else listed[0])).all(), counts[5]
 
 
 # Rows with no top-k cut (the open stage).  "peaked" logits are N(0, 6^2) (a
