@@ -62,6 +62,21 @@ class SpikingQwenConfig:
     threshold_init: float = 1.0
 
 
+def small_down_rows(hidden: int, inter: int) -> int:
+    """Rows up to which linear_decode takes the down projection ``[hidden,
+    inter]``; beyond, the library GEMM is as fast or faster.  Its column ranges
+    are one pass over the chip up to 256 rows for hidden <= 1024, up to 160 for hidden
+    <= 1536 (where 128 to 160 rows gain 3 %: left to the library).  Measured against the library GEMM (graph of 24 distinct weights,
+    us, 160 and 256 rows): 512 x 2816 5.9 / 7.3 and 6.0 / 7.4, 768 x 3072 6.1 / 7.7
+    and 7.0 / 8.4, 896 x 4864 8.9 / 10.9 and 11.1 / 11.2, 1024 x 4096 8.9 / 11.3 and
+    10.8 / 11.2, 1024 x 5120 11.0 / 13.1 and 13.4 / 13.8, but 1024 x 2816 6.9 / 7.9
+    and 8.4 / 8.2; 1280 x 5120 14.4 / 15.0 and 24.0 / 19.5, 1536 x 5120 14.6 / 15.1
+    and 26.4 / 19.6."""
+    if hidden <= 896 or (hidden <= 1024 and inter >= 4096):
+        return 256
+    return 160 if hidden <= 1024 else 128
+
+
 class _Layer:
     __slots__ = ("input_norm", "post_norm", "w_qkv", "b_qkv", "lif_qkv_beta", "lif_qkv_th",
                  "w_o", "w_gu", "lif_gate_beta", "lif_gate_th", "w_down", "w_gu_packed",
@@ -120,13 +135,9 @@ class SpikingDecoder:
         # The same batches run the q/k/v and o projections through
         # linear_decode (repacked copies of w_qkv, w_o); False keeps F.linear.
         # The down projection (long K) goes there up to small_down_max_rows rows
-        # (T * tokens).  With hidden <= 1024 all 256 rows are one pass over the
-        # chip (hidden 896, inter 4864: 128 rows 7.6 us against the library
-        # GEMM's 9.9, 160 rows 9.0 against 11.0, 192 and 256 rows equal at 10.9
-        # and 11.4); wider, the library GEMM is faster past 128 rows (256 rows,
-        # 1536 x 5120: 19.9 us against 27.1).
+        # (T * tokens).
         self.small_linear = True
-        self.small_down_max_rows = 256 if H <= 1024 else 128
+        self.small_down_max_rows = small_down_rows(H, I)
         # True folds each residual add + RMSNorm into the GEMM that consumes
         # its output (norm_linear_decode for q/k/v, norm_mlp_gate_lif for the
         # MLP): two launches fewer a layer, identical values, the residual

@@ -35,3 +35,14 @@ def test_pack_ref_and_unpack_ref_match_numpy_twins(C):
     back = unpack_ref(got, C, torch.float32)
     np.testing.assert_array_equal(back.numpy().astype(np.uint8), orc.np_unpack(got.numpy(), C))
     np.testing.assert_array_equal(back.numpy().astype(np.uint8), bits)
+
+
+@pytest.mark.parametrize("hidden,inter,rows", [
+    (512, 2816, 256), (896, 4864, 256), (1024, 4096, 256), (1024, 5120, 256),
+    (1024, 2816, 160),  # the library GEMM is 3 % faster from 176 rows on
+    (1280, 5120, 128), (1536, 5120, 128),
+])
+def test_down_projection_rows_follow_the_measurements(hidden, inter, rows):
+    from spikeinfer_amd.model import small_down_rows
+
+    assert small_down_rows(hidden, inter) == rows
