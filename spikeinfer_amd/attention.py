@@ -88,21 +88,18 @@ def _causal_offset_mask(query_len: int, total_len: int, device, dtype) -> torch.
     return torch.triu(mask, diagonal=ctx + 1)
 
 
-def _prefill_packed(q_packed, first, k_cache, v_cache, meta, out, head_dim, dtype):
+def _prefill_packed(q_packed, first, k_cache, v_cache, meta, out, head_dim):
     """Each prefill chunk attends to its sequence's whole cached prefix plus
     itself, straight from the packed words (spikeinfer/attention.py:161-178).
-    Row ``i`` of ``q_packed [T, n, H_q, W]`` is batch row ``first + i``; values
-    are rounded to ``dtype`` on the way to an ``out`` the kernel does not write."""
-    # (indexed: a list shorter than the others is an error)
-    chunks = [(meta.prefill_query_starts[i] - first, meta.prefill_query_starts[i], meta.prefill_query_lens[i],
-               meta.prefill_context_lens[i], meta.prefill_block_tables[i]) for i in range(meta.num_prefills)]
-    dst = out
-    if out.dtype not in PREFILL_DTYPES or out.stride(-1) != 1:  # (the kernel's outputs)
-        dst = torch.empty(out.shape, dtype=dtype, device=out.device)
-    paged_spike_attn_prefill(q_packed, k_cache, v_cache, chunks, dst, head_dim, meta.block_size)
-    if dst is not out:
-        for _, start, q_len, _, _ in chunks:
-            out[:, start:start + q_len] = dst[:, start:start + q_len]
+    Row ``i`` of ``q_packed [T, n, H_q, W]`` is batch row ``first + i``."""
+    starts, lens, ctxs, tables = (meta.prefill_query_starts, meta.prefill_query_lens, meta.prefill_context_lens,
+                                  meta.prefill_block_tables)
+    if min(len(starts), len(ctxs), len(tables)) < len(lens):
+        raise IndexError(f"{len(lens)} prefill chunks, but {len(starts)} starts, {len(ctxs)} context lengths and "
+                         f"{len(tables)} block tables")
+    chunks = [(start - first, start, q_len, ctx, table) for start, q_len, ctx, table in
+              zip(starts, lens, ctxs, tables)]
+    paged_spike_attn_prefill(q_packed, k_cache, v_cache, chunks, out, head_dim, meta.block_size)
 
 
 def _prefill(q_dense, k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim):
@@ -160,7 +157,7 @@ def paged_attention(
             num_kv_heads=num_kv_heads, out=out[:, :n_dec],
         )
     if packed:
-        _prefill_packed(q_words, 0, k_cache, v_cache, meta, out, head_dim, dtype)
+        _prefill_packed(q_words, 0, k_cache, v_cache, meta, out, head_dim)
     elif meta.num_prefills:
         _prefill(q_spk[:, 0], k_cache, v_cache, meta, out, num_q_heads, num_kv_heads, head_dim)
     return out.view(T, 1, n_tok, num_q_heads * head_dim)
@@ -202,9 +199,10 @@ def paged_attention_fused(
     """
     T, n_tok = q_cur.shape[0], q_cur.shape[1]
     dtype, device = q_cur.dtype, q_cur.device
-    if out is None:
+    given = out is not None
+    if not given:
         out = torch.empty((T, n_tok, num_q_heads, head_dim), device=device, dtype=dtype)
-    n_dec = meta.num_decode_tokens
+    n_dec, n_pre = meta.num_decode_tokens, meta.num_prefills
     # One launch for the LIF sites: k and v into their cache slots, the decode
     # tokens' q into the packed-query buffer, the prefill tokens' q into another.
     sites = [(k_cur, lif_k[0], lif_k[1], k_cache, True), (v_cur, lif_v[0], lif_v[1], v_cache, True)]
@@ -213,7 +211,7 @@ def paged_attention_fused(
             q_packed = torch.empty((T, n_dec, num_q_heads, packed_width(head_dim)),
                                    dtype=torch.int32, device=device)
         sites.append((q_cur[:, :n_dec], lif_q[0], lif_q[1], q_packed, False))
-    if meta.num_prefills:
+    if n_pre:
         q_words = torch.empty((T, n_tok - n_dec, num_q_heads, packed_width(head_dim)), dtype=torch.int32,
                               device=device)
         q_site = (q_cur[:, n_dec:], lif_q[0], lif_q[1], q_words, False)
@@ -228,6 +226,12 @@ def paged_attention_fused(
             head_dim=head_dim, block_size=meta.block_size, num_q_heads=num_q_heads,
             num_kv_heads=num_kv_heads, out=out[:, :n_dec],
         )
-    if meta.num_prefills:
-        _prefill_packed(q_words, n_dec, k_cache, v_cache, meta, out, head_dim, dtype)
+    if n_pre and given and (out.dtype not in PREFILL_DTYPES or out.stride(-1) != 1):
+        # not an output of the kernel: through one in the currents' type
+        dst = torch.empty(out.shape, dtype=dtype, device=device)
+        _prefill_packed(q_words, n_dec, k_cache, v_cache, meta, dst, head_dim)
+        for start, q_len in zip(meta.prefill_query_starts, meta.prefill_query_lens):
+            out[:, start:start + q_len] = dst[:, start:start + q_len]
+    elif n_pre:
+        _prefill_packed(q_words, n_dec, k_cache, v_cache, meta, out, head_dim)
     return out.view(T, 1, n_tok, num_q_heads * head_dim)
